@@ -25,7 +25,6 @@ constexpr int KPAD = 132;
 
 // LDS float offsets of the staged K/V rows (16-byte aligned for float4 stores)
 __host__ __device__ inline int seg_ks_off(int G) { return (G * 128 + 256 + G * SEG + 2 * G + 3) & ~3; }
-__host__ __device__ inline int rows_ks_off(int G) { return (G * 128 + G * SEG + 6 * G + 3) & ~3; }
 
 // max fold in the SUM64 pattern: a = (o > a ? o : a) with o the value of lane
 // l ^ d, d = 32, 16, 8, 4, 2, 1.

@@ -387,12 +387,15 @@ lq8_status launch_attention_seg(hipStream_t s, const AttnSegLaunch& a);
 lq8_status launch_attention_combine(hipStream_t s, const float* part, size_t part_stride, const int* d_pos,
                                     int batch, int num_heads, int cmax, float* out);
 
-// Prefill: one workgroup per (kv head, query row) over a filled cache.
+// Prefill: query rows over a filled cache; the outputs [n][num_heads * 128]
+// quantized into the GEMM operand layout (the values launch_quantize_act
+// gives for them; rows past n are not written).
 struct AttnRowsLaunch {
     const float* q_rows;   // [n][num_heads * 128] normalized, rotated
     const float* k_cache;
     const float* v_cache;
-    float* out;            // [n][num_heads * 128]
+    int8_t* codes;         // act_code_bytes(n, num_heads * 128)
+    uint32_t* scales;      // act_scale_bytes(n, num_heads * 128)
     int pos_base, n, num_heads, num_kv_heads, max_pos;
     float scale;
 };

@@ -55,6 +55,49 @@ __device__ __forceinline__ float expf_cr(float xf) {
     return (float)ldexp(p, (int)k);
 }
 
+// expf_cr's constants as a table: log2(e), ln2 high and low, 1/13!, 1/12!, .. 1/3!
+constexpr int EXP_CONSTS = 14;
+#define LQ8_EXP_CONSTS                                                                                           \
+    {1.4426950408889634074,  6.93147180369123816490e-01, 1.90821492927058770002e-10, 1.0 / 6227020800.0,         \
+     1.0 / 479001600.0,      1.0 / 39916800.0,           1.0 / 3628800.0,            1.0 / 362880.0,             \
+     1.0 / 40320.0,          1.0 / 5040.0,               1.0 / 720.0,                1.0 / 120.0,                \
+     1.0 / 24.0,             1.0 / 6.0}
+
+// x[i] = expf_cr(x[i]) for x <= 0 or NaN (differences to a maximum) without
+// branches and side by side (the chains are long): the same steps with k
+// rounded by adding 1.5 * 2^52 (its low word is then k), so that a NaN passes
+// through; what they give below -110 (-inf included) is replaced.  c: the
+// constants, as the caller holds them.
+template <int N, typename P>
+__device__ __forceinline__ void expf_le0(float (&x)[N], P c) {
+    double r[N], p[N];
+    int k[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const double xd = (double)x[i];
+        const double kk = xd * c[0] + 6755399441055744.0;
+        const double kd = kk - 6755399441055744.0;
+        k[i] = (int)(uint32_t)__builtin_bit_cast(uint64_t, kk);
+        r[i] = fma(-kd, c[1], xd);
+        r[i] = fma(-kd, c[2], r[i]);
+        p[i] = c[3];
+    }
+#pragma unroll
+    for (int j = 4; j < EXP_CONSTS; j++)
+#pragma unroll
+        for (int i = 0; i < N; i++) p[i] = fma(p[i], r[i], c[j]);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = fma(p[i], r[i], 0.5);
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = fma(p[i], r[i], 1.0);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        p[i] = fma(p[i], r[i], 1.0);
+        const float y = (float)ldexp(p[i], k[i]);
+        x[i] = x[i] < -110.0f ? 0.0f : y;
+    }
+}
+
 // Rust `f32 as i8`: saturating, NaN -> 0.
 __device__ __forceinline__ int sat_i8(float v) {
     if (v != v) return 0;

@@ -60,7 +60,7 @@ struct lq8_model {
     size_t tokens_cap = 0;
     // prefill buffers, capacity in rows
     size_t pf_cap = 0;
-    float *P_h = nullptr, *P_x = nullptr, *P_qkv = nullptr, *P_qr = nullptr, *P_attn = nullptr, *P_gu = nullptr,
+    float *P_h = nullptr, *P_x = nullptr, *P_qkv = nullptr, *P_qr = nullptr, *P_gu = nullptr,
           *P_xs = nullptr;
     int8_t* P_xq = nullptr;
     // replayed decode steps, indexed by the token they forward: [0] the token
@@ -142,7 +142,7 @@ void release(lq8_model* m) {
     F(m->cos_t); F(m->sin_t); F(m->kc); F(m->vc);
     F(m->h); F(m->h2); F(m->qkv); F(m->gu); F(m->apart); F(m->logits); F(m->arg_val); F(m->arg_idx); F(m->dpart);
     F(m->d_ids); F(m->d_pos); F(m->d_step); F(m->d_tok); F(m->d_tokens);
-    F(m->P_h); F(m->P_x); F(m->P_qkv); F(m->P_qr); F(m->P_attn); F(m->P_gu); F(m->P_xs); F(m->P_xq);
+    F(m->P_h); F(m->P_x); F(m->P_qkv); F(m->P_qr); F(m->P_gu); F(m->P_xs); F(m->P_xq);
     F(m->d_scfg); F(m->d_counts); F(m->s_work);
     F(m->d_player); F(m->hand); F(m->d_pargs); F(m->d_abort);
     delete m;
@@ -276,7 +276,7 @@ lq8_status ensure_prefill(lq8_model* m, size_t n) {
     if (n <= m->pf_cap) return LQ8_OK;
     LQ8_HIP(hipStreamSynchronize(m->ctx->stream));
     auto F = [](float*& p) { if (p) (void)hipFree(p); p = nullptr; };
-    F(m->P_h); F(m->P_x); F(m->P_qkv); F(m->P_qr); F(m->P_attn); F(m->P_gu); F(m->P_xs);
+    F(m->P_h); F(m->P_x); F(m->P_qkv); F(m->P_qr); F(m->P_gu); F(m->P_xs);
     if (m->P_xq) (void)hipFree(m->P_xq);
     m->P_xq = nullptr;
     m->pf_cap = 0;
@@ -284,7 +284,7 @@ lq8_status ensure_prefill(lq8_model* m, size_t n) {
     const int kmax = (int)std::max(Hd, std::max(m->QD, (size_t)I));
     lq8_status st;
     if ((st = dalloc(&m->P_h, n * Hd)) || (st = dalloc(&m->P_x, n * Hd)) || (st = dalloc(&m->P_qkv, n * m->QKV)) ||
-        (st = dalloc(&m->P_qr, n * m->QD)) || (st = dalloc(&m->P_attn, n * m->QD)) ||
+        (st = dalloc(&m->P_qr, n * m->QD)) ||
         (st = dalloc(&m->P_gu, n * 2 * I)) ||
         (st = dalloc(&m->P_xs, act_scale_bytes((int)n, kmax) / sizeof(float))) ||
         (st = dalloc(&m->P_xq, act_code_bytes((int)n, kmax))))
@@ -428,10 +428,12 @@ lq8_status enqueue_prefill(lq8_model* m, int n, int pos_base, float* trace = nul
                         m->vc + l * layer_kv, nullptr, pos_base, n, (int)c.num_heads, (int)c.num_kv_heads,
                         (int)c.head_dim, (int)c.max_positions, c.rms_norm_eps};
         if ((st = launch_qk_rope_kv(s, qr))) return st;
-        AttnRowsLaunch at{m->P_qr, m->kc + l * layer_kv, m->vc + l * layer_kv, m->P_attn, pos_base, n,
-                          (int)c.num_heads, (int)c.num_kv_heads, (int)c.max_positions, scale};
+        AttnRowsLaunch at{m->P_qr, m->kc + l * layer_kv, m->vc + l * layer_kv, m->P_xq,
+                          reinterpret_cast<uint32_t*>(m->P_xs), pos_base, n, (int)c.num_heads, (int)c.num_kv_heads,
+                          (int)c.max_positions, scale};
         if ((st = launch_attention_rows(s, at))) return st;
-        if ((st = quant_gemm(m, m->P_attn, n, L.o, m->P_h, m->P_h))) return st;
+        if ((st = launch_gemm(s, m->P_xq, reinterpret_cast<const uint32_t*>(m->P_xs), n, L.o, m->P_h, m->P_h)))
+            return st;
         if ((st = norm_quant_gemm(m, m->P_h, L.post_norm, n, L.gu, m->P_gu))) return st;
         if ((st = launch_silu_quantize_act(s, m->P_gu, n, I, m->P_xq, reinterpret_cast<uint32_t*>(m->P_xs))))
             return st;

@@ -11,6 +11,8 @@
 //           (m, num, den) update m' = max(m, m_c), a = exp(m - m'),
 //           b = exp(m_c - m'), num = num a + b o_c, den = den a + b l_c; the
 //           output is num / den.
+#include <type_traits>
+
 #include "attn_device.h"
 #include "lq8_internal.h"
 #include "lq8_numerics.h"
@@ -179,114 +181,304 @@ __global__ __launch_bounds__(128) void k_attn_combine(const float* __restrict__ 
     out[(size_t)b * H * 128 + h * 128 + d] = __fdiv_rn(num, den);
 }
 
-// Attention over n query rows with a filled cache (prefill): one workgroup
-// per (kv head, R consecutive rows), R * G <= 16.  The segments run in order
-// with the running update; each K/V segment is staged once for the R rows,
-// and a row whose positions end before a segment skips it (its arithmetic is
-// the single-row sequence exactly).
-template <int R>
-__global__ __launch_bounds__(ATT_THREADS) void k_attn_rows(AttnRowsLaunch a) {
-    extern __shared__ float sm[];
-    const int kvh = blockIdx.x, i0 = blockIdx.y * R;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int G = a.num_heads / a.num_kv_heads, RG = R * G;
+// Attention over n query rows with a filled cache (prefill), its output
+// quantized into the o projection's operand.  One workgroup of 4 waves per (kv
+// head, NV = 16 NVT query vectors): vector v is query head v % G of row i0 +
+// v / G.  The 64-position segments run in order, one per step, with the
+// running update of each vector.
+//
+// The chains round every product before it is added, so a multiply-accumulate
+// is no fma; the matrix cores take the products: v_mfma_f32_16x16x1_4b_f32
+// with C = 0 gives four 16 x 16 outer products, each element round(a * b)
+// exactly as v_mul_f32 rounds it (subnormals included; a zero product is +0
+// instead of -0, which no sum that starts from +0 can tell), at twice the
+// VALU's rate, and the VALU only adds them in the order of the chain.  Operand
+// lane l is row (column) l % 16 of block l / 16, and the blocks are four terms
+// of the chain: a float4 of 16 consecutive terms per lane group feeds 4
+// instructions (component c, block p: term 4 p + c), whose 64 products per
+// lane are then added term by term.  Result lane l holds column l % 16, rows
+// 4 (l / 16) .. + 3 of every block.
+//   scores  rows = 16 keys (wave w: keys 16 w .. of the segment, straight from
+//           the cache), columns = 16 query vectors (LDS), terms = d
+//   P.V     rows = 16 d (wave w: d 32 w .. + 31, even and odd d as two tiles),
+//           columns = 16 query vectors, terms = the segment's 64 positions
+//   softmax a thread takes 4 NVT positions of one vector, part + PARTS i, so
+//           that SUM64's distances >= PARTS are sums inside the thread
+//   output  a wave's 32 d of a vector are one Q8_0 block of the operand
+// Positions past a row's own enter P.V with e = 0; their products are zeros
+// unless V is not finite there, and a segment where that is so takes the adds
+// one by one under the row's length.
+//
+// Bound: instruction issue.  At 2048 rows (Qwen3-0.6B) the VALU instructions
+// (758k cycles per SIMD, 540k of them the chains' adds) and the f32 matrix
+// instructions (270k; they use the same fp32 units, and issuing the next
+// group's products between a group's adds changed nothing) fill the 1.0M
+// cycles the kernel runs.  Against one chain per thread from LDS followed by
+// the separate quantizer: 1283 -> 423 us at 2048 rows, 370 -> 128 at 1024, 109
+// -> 48 at 512, 20 -> 15 at 128 (where a wave's chain latencies bound it), and
+// 5 us of quantizer less.  64 vectors per workgroup (256 VGPRs) measured 553
+// us at 2048 rows.
+typedef float v16f __attribute__((ext_vector_type(16)));
+constexpr int AR_THREADS = 256;
+constexpr int AR_QPAD = 132, AR_SPAD = 68;  // LDS row strides: 16-byte aligned, 4 banks apart
+
+// exp's constants in memory: read by scalar loads where they are used (as
+// literals in a loop they are hoisted into 26 VGPRs)
+__constant__ const double exp_consts[EXP_CONSTS] = LQ8_EXP_CONSTS;
+typedef const double __attribute__((address_space(4))) * ExpConsts;
+__device__ __forceinline__ ExpConsts exp_consts_here() {
+    ExpConsts c = (ExpConsts)exp_consts;
+    asm volatile("" : "+s"(c));
+    return c;
+}
+
+__device__ __forceinline__ v16f products(float a, float b) {
+    const v16f z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, z, 0, 0, 0);
+}
+
+// s[v] += the 16 terms of (a, b) in order; MASKED: only terms j0 + t < nj.
+// The empty asm statements keep one group's 64 products in registers at a
+// time (a pure value is otherwise computed at its use).
+template <bool MASKED>
+__device__ __forceinline__ void add_terms(const float (&a)[4], float4 b, float (&s)[4], int j0, int nj) {
+    asm volatile("" : "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w));
+    const v16f p0 = products(a[0], b.x), p1 = products(a[1], b.y), p2 = products(a[2], b.z), p3 = products(a[3], b.w);
+#pragma unroll
+    for (int p = 0; p < 4; p++) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const v16f& q = c == 0 ? p0 : c == 1 ? p1 : c == 2 ? p2 : p3;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float t = s[v] + q[4 * p + v];
+                s[v] = !MASKED || j0 + 4 * p + c < nj ? t : s[v];
+            }
+        }
+    }
+    asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// 8 codes of a Q8_0 block as the two dwords of its operand bytes
+__device__ __forceinline__ uint2 codes8(const float (&y)[8], float id) {
+    uint32_t w[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        w[i] = (uint32_t)(quant_code(y[4 * i], id) & 0xFF) | ((uint32_t)(quant_code(y[4 * i + 1], id) & 0xFF) << 8) |
+               ((uint32_t)(quant_code(y[4 * i + 2], id) & 0xFF) << 16) | ((uint32_t)(quant_code(y[4 * i + 3], id) & 0xFF) << 24);
+    return make_uint2(w[0], w[1]);
+}
+
+template <int NVT>
+__global__ __launch_bounds__(AR_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_rows(AttnRowsLaunch a) {
+    constexpr int NV = 16 * NVT, PARTS = AR_THREADS / NV, KPT = SEG / PARTS;
+    __shared__ __attribute__((aligned(16))) float qs[NV * AR_QPAD];
+    __shared__ __attribute__((aligned(16))) float sbuf[2][NV * AR_SPAD];  // scores, then exps
+    __shared__ float coef[2][NV * 2];                                     // the step's a, b of each vector
+    __shared__ float dens[NV];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, p = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = a.num_heads / a.num_kv_heads, R = NV / G;
     const int QD = a.num_heads * 128;
+    // the rows with the most positions first
+    const int kvh = blockIdx.x, i0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * R;
     const int nr = min(R, a.n - i0);
-    const int Lmax = a.pos_base + i0 + nr;  // positions of the workgroup's last row
+    const int L0 = a.pos_base + i0 + 1;   // positions of the first row
+    const int Lmax = L0 + nr - 1;         // and of the last
     const float* Kc = a.k_cache + (size_t)kvh * a.max_pos * 128;
     const float* Vc = a.v_cache + (size_t)kvh * a.max_pos * 128;
-    float* qs = sm;                      // [R][G][128]
-    float* sc = qs + RG * 128;           // [R][G][64]
-    float* mlc = sc + RG * SEG;          // [R][G][2]
-    float* run = mlc + 2 * RG;           // [R][G][4]: m, den, a, b
-    float* ks = sm + rows_ks_off(RG);    // [64][KPAD], later vs [64][128]
-    for (int e = tid; e < RG * 128; e += ATT_THREADS) {
-        const int rr = e / (G * 128), w = e - rr * G * 128;
-        qs[e] = a.q_rows[(size_t)(i0 + min(rr, nr - 1)) * QD + kvh * G * 128 + w];
-    }
-    for (int h = tid; h < RG; h += ATT_THREADS) {
-        run[4 * h] = -__builtin_huge_valf();
-        run[4 * h + 1] = 0.0f;
-    }
-    // thread t < R * G * 128 (looping) keeps num for (row, head, d) = (t / (G * 128), (t / 128) % G, t % 128)
-    constexpr int MAXR = 16 * 128 / ATT_THREADS;
-    float num[MAXR];
+    float4 kr[8];
+    float2 vr[4][4];
+    // a whole segment loads from a uniform base with constant lane offsets; in
+    // the last one the rows past the last row's position read that row
+    const unsigned ko = ((16 * w + r) * 128 + 4 * p) * 4, vo = (4 * p * 128 + 32 * w + 2 * r) * 4;
+    auto load_k = [&](int js) {
+        if (js + SEG <= Lmax) {
+            const char* kp = (const char*)(Kc + (size_t)js * 128);
 #pragma unroll
-    for (int r = 0; r < MAXR; r++) num[r] = 0.0f;
-    float4 kreg[ATT_F4], vreg[ATT_F4];
-    for (int js = 0; js < Lmax; js += SEG) {
-        const int njmax = min(SEG, Lmax - js);
-        seg_load(Kc, Vc, js, njmax, kreg, vreg);
-        __syncthreads();
+            for (int i = 0; i < 8; i++) kr[i] = *(const float4*)(kp + ko + 64 * i);
+        } else if (js < Lmax) {
+            const float* kp = Kc + (size_t)min(js + 16 * w + r, Lmax - 1) * 128 + 4 * p;
 #pragma unroll
-        for (int u = 0; u < ATT_F4; u++) {
-            const int f = tid + u * ATT_THREADS;
-            const int j = f >> 5, c4 = f & 31;
-            if (j < njmax) {
-                *(float4*)(ks + j * KPAD + c4 * 4) = kreg[u];
-            }
+            for (int i = 0; i < 8; i++) kr[i] = *(const float4*)(kp + 16 * i);
         }
-        __syncthreads();
-        // scores q.k, sequential over d, then times the scale (one thread per (row, head, position))
-        for (int t = tid; t < RG * SEG; t += ATT_THREADS) {
-            const int rh = t / SEG, j = t - rh * SEG, rr = rh / G;
-            const int nj = min(SEG, a.pos_base + i0 + rr + 1 - js);
-            if (rr < nr && j < nj) sc[rh * SEG + j] = qk_dot128(qs + rh * 128, ks + j * KPAD) * a.scale;
-        }
-        __syncthreads();
-        // segment softmax per (row, head): max, exp, SUM64 denominator
-        for (int rh = wave; rh < RG; rh += ATT_THREADS / 64) {
-            const int rr = rh / G;
-            const int nj = min(SEG, a.pos_base + i0 + rr + 1 - js);
-            if (rr < nr && nj > 0) {
-                const float sv = lane < nj ? sc[rh * SEG + lane] : -__builtin_huge_valf();
-                const float mc = wave_max64(sv);
-                const float e = lane < nj ? expf_cr(sv - mc) : 0.0f;
-                const float lc = wave_sum64(e);
-                if (lane < nj) sc[rh * SEG + lane] = e;
-                if (lane == 0) {
-                    mlc[2 * rh] = mc;
-                    mlc[2 * rh + 1] = lc;
-                }
-            }
-        }
-        __syncthreads();
-        for (int rh = tid; rh < RG; rh += ATT_THREADS) {
-            const int rr = rh / G;
-            if (rr < nr && a.pos_base + i0 + rr + 1 - js > 0) {
-                const float m = run[4 * rh], mc = mlc[2 * rh];
-                const float mn = m > mc ? m : mc;
-                const float ea = expf_cr(m - mn), eb = expf_cr(mc - mn);
-                run[4 * rh] = mn;
-                run[4 * rh + 1] = run[4 * rh + 1] * ea + eb * mlc[2 * rh + 1];
-                run[4 * rh + 2] = ea;
-                run[4 * rh + 3] = eb;
-            }
-        }
-        seg_stage_v(vreg, njmax, -1, nullptr, ks);
-        __syncthreads();
+    };
+    auto load_v = [&](int js) {
+        if (js + SEG <= Lmax) {
+            const char* vp = (const char*)(Vc + (size_t)js * 128);
 #pragma unroll
-        for (int r = 0; r < MAXR; r++) {
-            const int t = tid + r * ATT_THREADS;
-            if (t < RG * 128) {
-                const int rh = t >> 7, d = t & 127, rr = rh / G;
-                const int nj = min(SEG, a.pos_base + i0 + rr + 1 - js);
-                if (rr < nr && nj > 0) {
-                    const float o = pv_chain(sc + rh * SEG, ks, d, nj);
-                    num[r] = num[r] * run[4 * rh + 2] + run[4 * rh + 3] * o;
-                }
-            }
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) vr[i][c] = *(const float2*)(vp + 16 * 512 * i + vo + 512 * c);
+        } else if (js < Lmax) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    vr[i][c] = *(const float2*)(Vc + (size_t)min(js + 16 * i + 4 * p + c, Lmax - 1) * 128 + 32 * w + 2 * r);
         }
+    };
+    load_k(0);
+    for (int e = tid; e < NV * 32; e += AR_THREADS) {
+        const int v = e >> 5, c4 = e & 31, rr = min(v / G, nr - 1), h = v % G;  // spare vectors repeat the last row
+        *(float4*)(qs + v * AR_QPAD + 4 * c4) =
+            *(const float4*)(a.q_rows + (size_t)(i0 + rr) * QD + (kvh * G + h) * 128 + 4 * c4);
     }
+    load_v(0);
+    int lenv[NVT];  // positions of the lane's column vectors
+    float num[NVT][2][4];
+#pragma unroll
+    for (int vt = 0; vt < NVT; vt++) {
+        lenv[vt] = L0 + min((16 * vt + r) / G, nr - 1);
+#pragma unroll
+        for (int v = 0; v < 4; v++) num[vt][0][v] = num[vt][1][v] = 0.0f;
+    }
+    const int sv = tid / PARTS, part = tid % PARTS;  // this thread's softmax vector
+    const int slen = L0 + min(sv / G, nr - 1);
+    float mrun = -__builtin_huge_valf(), den = 0.0f;
     __syncthreads();
+    int buf = 0;
+    for (int js = 0; js < Lmax; js += SEG, buf ^= 1) {
+        float* S = sbuf[buf];
+        const bool full = js + SEG <= L0;  // every row has the whole segment
+        // scores of the wave's 16 keys
 #pragma unroll
-    for (int r = 0; r < MAXR; r++) {
-        const int t = tid + r * ATT_THREADS;
-        if (t < RG * 128) {
-            const int rh = t >> 7, d = t & 127, rr = rh / G, h = rh - rr * G;
-            if (rr < nr)
-                a.out[(size_t)(i0 + rr) * QD + (kvh * G + h) * 128 + d] = __fdiv_rn(num[r], run[4 * rh + 1]);
+        for (int vt = 0; vt < NVT; vt++) {
+            float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            const float* qp = qs + (16 * vt + r) * AR_QPAD + 4 * p;
+            float4 q = *(const float4*)qp;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float ka[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
+                const float4 qn = *(const float4*)(qp + 16 * min(i + 1, 7));  // the next group's, ahead of the adds
+                add_terms<false>(ka, q, s, 0, 0);
+                q = qn;
+            }
+            *(float4*)(S + (16 * vt + r) * AR_SPAD + 16 * w + 4 * p) =
+                make_float4(s[0] * a.scale, s[1] * a.scale, s[2] * a.scale, s[3] * a.scale);
+        }
+        load_k(js + SEG);
+        lds_sync();
+        {
+            // m_c, e, l_c of the thread's vector, then its running update
+            const ExpConsts ec = exp_consts_here();
+            const int nj = min(SEG, slen - js);
+            float* row = S + sv * AR_SPAD + part;
+            float x[KPT + 1];  // the thread's scores and the update's exponent
+            float mc = -__builtin_huge_valf();
+#pragma unroll
+            for (int i = 0; i < KPT; i++) x[i] = row[PARTS * i];
+            if (!full) {
+#pragma unroll
+                for (int i = 0; i < KPT; i++) x[i] = part + PARTS * i < nj ? x[i] : -__builtin_huge_valf();
+            }
+#pragma unroll
+            for (int i = 0; i < KPT; i++) mc = fmaxf(mc, x[i]);
+            mc = fmaxf(mc, lane_xor<1>(mc));
+            mc = fmaxf(mc, lane_xor<2>(mc));
+            if (PARTS > 4) mc = fmaxf(mc, lane_xor<4>(mc));
+            if (PARTS > 8) mc = fmaxf(mc, lane_xor<8>(mc));
+#pragma unroll
+            for (int i = 0; i < KPT; i++) x[i] = x[i] - mc;
+            if (!full) {
+                // (a row with no position here has mc = -inf)
+#pragma unroll
+                for (int i = 0; i < KPT; i++) x[i] = part + PARTS * i < nj ? x[i] : -__builtin_huge_valf();
+            }
+            const float mn = mrun > mc ? mrun : mc;
+            x[KPT] = (part & 1 ? mc : mrun) - mn;
+            expf_le0(x, ec);
+#pragma unroll
+            for (int i = 0; i < KPT; i++) row[PARTS * i] = x[i];
+#pragma unroll
+            for (int d = KPT / 2; d > 0; d /= 2)
+#pragma unroll
+                for (int i = 0; i < d; i++) x[i] = x[i] + x[i + d];
+            float lc = x[0];
+            if (PARTS > 8) lc = lc + lane_xor<8>(lc);
+            if (PARTS > 4) lc = lc + lane_xor<4>(lc);
+            lc = lc + lane_xor<2>(lc);
+            lc = lc + lane_xor<1>(lc);
+            const float ex = x[KPT], ey = lane_xor<1>(ex);
+            if (part < 2) coef[buf][2 * sv + part] = ex;
+            const float dn = (part & 1 ? den * ey : den * ex) + (part & 1 ? ex * lc : ey * lc);
+            den = nj > 0 ? dn : den;
+            mrun = nj > 0 ? mn : mrun;
+        }
+        lds_sync();
+        // WHOLE: the step is full; M: V is not finite somewhere in the segment
+        auto pv = [&](auto whole, auto masked) {
+            constexpr bool WHOLE = decltype(whole)::value, M = decltype(masked)::value;
+#pragma unroll
+            for (int vt = 0; vt < NVT; vt++) {
+                float o[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+                const int nj = lenv[vt] - js;
+                const float* ep = S + (16 * vt + r) * AR_SPAD + 4 * p;
+                float4 e = *(const float4*)ep;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (!WHOLE && js + 16 * i >= Lmax) break;  // no row has these positions
+                    const float4 en = *(const float4*)(ep + 16 * min(i + 1, 3));
+                    const float v0[4] = {vr[i][0].x, vr[i][1].x, vr[i][2].x, vr[i][3].x};
+                    const float v1[4] = {vr[i][0].y, vr[i][1].y, vr[i][2].y, vr[i][3].y};
+                    add_terms<M>(v0, e, o[0], 16 * i, nj);
+                    add_terms<M>(v1, e, o[1], 16 * i, nj);
+                    e = en;
+                }
+                const float ca = coef[buf][2 * (16 * vt + r)], cb = coef[buf][2 * (16 * vt + r) + 1];
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const float y = num[vt][t][v] * ca + cb * o[t][v];
+                        num[vt][t][v] = WHOLE || nj > 0 ? y : num[vt][t][v];
+                    }
+            }
+        };
+        if (full) {
+            pv(std::true_type{}, std::false_type{});
+        } else {
+            uint32_t top = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    top = max(top, __float_as_uint(vr[i][c].x) & 0x7FFFFFFFu);
+                    top = max(top, __float_as_uint(vr[i][c].y) & 0x7FFFFFFFu);
+                }
+            if (__all(top < 0x7F800000u)) pv(std::false_type{}, std::false_type{});
+            else pv(std::false_type{}, std::true_type{});
+        }
+        load_v(js + SEG);
+    }
+    if (part == 0) dens[sv] = den;
+    __syncthreads();
+    // lane (r, p): values 8 p .. + 7 of block 4 head + w of vector 16 vt + r
+    const int nb = a.num_heads * 4, np = nb / 2, nbp4 = 2 * ((nb + GEMM_GROUP - 1) / GEMM_GROUP);
+#pragma unroll
+    for (int vt = 0; vt < NVT; vt++) {
+        const int v = 16 * vt + r, rr = v / G, head = kvh * G + v - rr * G, row = i0 + rr;
+        const float dn = dens[v];
+        float y[8], amax = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            y[i] = __fdiv_rn(num[vt][i & 1][i >> 1], dn);
+            amax = fmaxf(amax, fabsf(y[i]));
+        }
+        amax = fmaxf(amax, lane_xor<16>(amax));
+        amax = fmaxf(amax, lane_xor<32>(amax));
+        const QBlock qb = block_scale(amax);
+        const uint2 c = codes8(y, block_inv(qb.d));
+        if (rr < nr) {  // (not the spare vectors)
+            const int b = head * 4 + w;
+            *(uint2*)(a.codes + code_off(row / TILE_ROWS, np, b, p >> 1, row % TILE_ROWS) + 8 * (p & 1)) = c;
+            if ((p & 1) == 0) {
+                uint32_t* xs = a.scales + ((size_t)((row >> 5) * nbp4 + (b >> 2)) * 64 + 16 * p + (row & 31)) * 4;
+                xs[w] = p ? 0u : qb.d16;
+                // an odd head count: the operand's last 4 blocks are padding
+                if (w == 3 && head == a.num_heads - 1 && (nb >> 2) < nbp4) *(uint4*)(xs + 256) = make_uint4(0, 0, 0, 0);
+            }
         }
     }
 }
@@ -376,7 +568,6 @@ constexpr int ATT_WG_TARGET = 512;  // decode attention workgroups sought per la
 constexpr int ATT_MIN_SLOTS = 8;    // segment slots at least (512 positions without a second round)
 
 size_t seg_smem(int G) { return ((size_t)seg_ks_off(G) + (size_t)SEG * KPAD) * sizeof(float); }
-size_t rows_smem(int G) { return ((size_t)rows_ks_off(G) + (size_t)SEG * KPAD) * sizeof(float); }
 
 }  // namespace
 
@@ -428,12 +619,15 @@ lq8_status launch_attention_rows(hipStream_t s, const AttnRowsLaunch& a) {
     if (!attention_supported(a.num_heads, a.num_kv_heads, 128))
         return fail(LQ8_ERR_SHAPE_MISMATCH, "attention: unsupported head layout");
     const int G = a.num_heads / a.num_kv_heads;
-    // rows per workgroup: R * G <= 16 (the per-thread output registers)
-    const int R = G <= 4 ? 4 : G <= 8 ? 2 : 1;
-    const dim3 grid((unsigned)a.num_kv_heads, (unsigned)((a.n + R - 1) / R));
-    if (R == 4) hipLaunchKernelGGL(k_attn_rows<4>, grid, dim3(ATT_THREADS), rows_smem(R * G), s, a);
-    else if (R == 2) hipLaunchKernelGGL(k_attn_rows<2>, grid, dim3(ATT_THREADS), rows_smem(R * G), s, a);
-    else hipLaunchKernelGGL(k_attn_rows<1>, grid, dim3(ATT_THREADS), rows_smem(R * G), s, a);
+    // 32 query vectors per workgroup where that still leaves four workgroups a
+    // CU (the per-step work is shared by more rows: 430 against 462 us at 2048
+    // rows of Qwen3-0.6B), else 16 (the rows' lengths balance better: 133
+    // against 159 us at 1024 rows, 48 against 73 at 512)
+    auto tiles = [&](int nv) { return (a.n + nv / G - 1) / (nv / G); };
+    const bool two = a.num_kv_heads * tiles(32) >= 1024;
+    const dim3 grid((unsigned)a.num_kv_heads, (unsigned)tiles(two ? 32 : 16));
+    if (two) hipLaunchKernelGGL(k_attn_rows<2>, grid, dim3(AR_THREADS), 0, s, a);
+    else hipLaunchKernelGGL(k_attn_rows<1>, grid, dim3(AR_THREADS), 0, s, a);
     LQ8_HIP(hipGetLastError());
     return LQ8_OK;
 }
