@@ -74,18 +74,25 @@ struct lq8_moe {
 namespace {
 
 // ---- router ------------------------------------------------------------------
-// One workgroup of 16 waves for the batch.  Wave w routes tokens w, w + 16,
-// ...: lane l holds scores l, l + 64, ...; m = max (exact in any order),
-// e = exp(s - m), S = SUM64(e) (lane l adds its entries in order, then the
-// xor fold), p = e / S.  An entry's rank is the number of entries with a
-// larger p or an equal p and a lower index; ranks below top_k are chosen, in
-// rank order; weights p_r / (((p_0 + p_1) + p_2) + ...).  Then the routed
-// (token, rank) slots t * top_k + r are counted per expert, the active
-// experts numbered by descending vector count, then ascending index (n_act,
-// act_e, vbeg, vcnt; the expert GEMVs' workgroups follow that order), and
-// each slot placed in its expert's list (slots, by ascending expert).  The order inside one expert's
-// list is whatever the atomics give: every slot is computed on its own, so
-// results do not depend on it.
+// One workgroup of 16 waves for the batch of a layer.  Wave w routes tokens w,
+// w + 16, ...: lane l holds scores l, l + 64, ... (NJ of them); m = max (exact
+// in any order), e = exp(s - m), S = SUM64(e) (lane l adds its entries in
+// order, then the xor fold), p = e / S.  The experts are picked rank by rank:
+// the wave's largest p (its bits, as integers), the lowest index among equals
+// (a ballot per entry), that entry out of the next rounds; weights
+// p_r / (((p_0 + p_1) + p_2) + ...).  Then (lists: only the batched experts'
+// kernels read them) the routed (token, rank) slots t * top_k + r are counted
+// per expert, the active experts numbered by descending vector count, then
+// ascending index (n_act, act_e, vbeg, vcnt; the expert GEMVs' workgroups
+// follow that order), and each slot placed in its expert's list (slots, by
+// ascending expert).  The order inside one expert's list is whatever the
+// atomics give: every slot is computed on its own, so results do not depend on
+// it.
+// One CU does a layer's routing, so instructions and serial LDS reads bound
+// it: picking by rounds (about 25 instructions per rank) instead of ranking
+// every entry against every other, and the numbering by 4 threads per expert
+// with 16-byte reads instead of one thread per 4 experts, took two layers of
+// 128 experts, top 8, from 66 to 11 us at 32 tokens and from 31 to 3.3 us at one.
 constexpr int ROUTE_WAVES = 16;
 struct RouteArgs {
     const float* scores;  // [layers][T][E]
@@ -97,12 +104,13 @@ struct RouteArgs {
     int* vbeg;            // [layers][E]
     int* vcnt;            // [layers][E]
     int* slots;           // [layers][B * K]
+    int lists;            // 0: rids and rw only
 };
+template <int NJ>
 __global__ __launch_bounds__(64 * ROUTE_WAVES) void k_moe_route(RouteArgs ra) {
-    __shared__ float4 sp4[ROUTE_WAVES][MOE_MAX_EXPERTS / 4];
-    __shared__ float selp[ROUTE_WAVES][MOE_MAX_TOPK];
     __shared__ int sid[MOE_MAX_BATCH * MOE_MAX_TOPK];
-    __shared__ int cnt[MOE_MAX_EXPERTS], beg[MOE_MAX_EXPERTS], fill[MOE_MAX_EXPERTS];
+    __shared__ __attribute__((aligned(16))) int cnt[MOE_MAX_EXPERTS];
+    __shared__ int beg[MOE_MAX_EXPERTS], fill[MOE_MAX_EXPERTS];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const float NEG = -__builtin_huge_valf();
@@ -114,17 +122,15 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void k_moe_route(RouteArgs ra) {
     int* __restrict__ vbeg = ra.vbeg + (size_t)l * E;
     int* __restrict__ vcnt = ra.vcnt + (size_t)l * E;
     int* __restrict__ slots = ra.slots + (size_t)l * ra.B * K;
-    float* sp = (float*)sp4[wave];
-    const int E16 = (E + 15) & ~15;  // the rank loop reads 16 entries at a time; padding is -inf
-    for (int e = tid; e < E; e += 64 * ROUTE_WAVES) {
-        cnt[e] = 0;
-        fill[e] = 0;
+    if (tid < MOE_MAX_EXPERTS) {
+        cnt[tid] = 0;
+        fill[tid] = 0;
     }
     for (int t = wave; t < T; t += ROUTE_WAVES) {
-        float p[4];
+        float p[NJ];
         float m = NEG;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < NJ; j++) {
             const int i = lane + 64 * j;
             p[j] = i < E ? scores[(size_t)t * E + i] : NEG;
             m = fmaxf(m, p[j]);
@@ -137,62 +143,52 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void k_moe_route(RouteArgs ra) {
         m = fmaxf(m, lane_xor<1>(m));
         float acc = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < NJ; j++) {
             if (lane + 64 * j < E) {
                 p[j] = expf_cr(p[j] - m);
                 acc = acc + p[j];
             }
         }
         acc = wave_sum64(acc);
+        // p >= 0, so its bits order as integers; -1: no entry, or picked
+        int key[NJ];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = lane + 64 * j;
-            if (i < E) p[j] = __fdiv_rn(p[j], acc);
-            if (i < E16) sp[i] = p[j];  // NEG past E
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        // rank = entries with a larger p, or an equal p and a lower index
-        int rank[4] = {0, 0, 0, 0};
-        for (int i0 = 0; i0 < E16; i0 += 16) {
-            float4 q4[4];
+        for (int j = 0; j < NJ; j++)
+            key[j] = lane + 64 * j < E ? __float_as_int(__fdiv_rn(p[j], acc)) & 0x7FFFFFFF : -1;
+        float mine = 0.0f, tot = 0.0f;  // lane r: p of rank r
+        int id = 0;
+        for (int r = 0; r < K; r++) {
+            int best = key[0];
 #pragma unroll
-            for (int u = 0; u < 4; u++) q4[u] = sp4[wave][(i0 >> 2) + u];
+            for (int j = 1; j < NJ; j++) best = max(best, key[j]);
+            best = max(best, lane_xor_int<32>(best));
+            best = max(best, lane_xor_int<16>(best));
+            best = max(best, lane_xor_int<8>(best));
+            best = max(best, lane_xor_int<4>(best));
+            best = max(best, lane_xor_int<2>(best));
+            best = max(best, lane_xor_int<1>(best));
+            int win = -1;
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float q[4] = {q4[u].x, q4[u].y, q4[u].z, q4[u].w};
+            for (int j = 0; j < NJ; j++) {
+                const unsigned long long eq = __ballot(key[j] == best);
+                if (win < 0 && eq) win = 64 * j + __ffsll(eq) - 1;
+            }
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int i2 = i0 + 4 * u + c;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int i = lane + 64 * j;
-                        rank[j] += (q[c] > p[j] || (q[c] == p[j] && i2 < i)) ? 1 : 0;
-                    }
-                }
+            for (int j = 0; j < NJ; j++)
+                if (lane + 64 * j == win) key[j] = -1;
+            tot = tot + __int_as_float(best);
+            if (lane == r) {
+                mine = __int_as_float(best);
+                id = win;
             }
         }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int i = lane + 64 * j;
-            if (i < E && rank[j] < K) {
-                selp[wave][rank[j]] = p[j];
-                rids[t * K + rank[j]] = (uint32_t)i;
-                sid[t * K + rank[j]] = i;
-            }
+        if (lane < K) {
+            rids[t * K + lane] = (uint32_t)id;
+            sid[t * K + lane] = id;
+            rw[t * K + lane] = __fdiv_rn(mine, tot);
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        float pk[MOE_MAX_TOPK];
-#pragma unroll
-        for (int r = 0; r < MOE_MAX_TOPK; r++) pk[r] = r < K ? selp[wave][r] : 0.0f;
-        float tot = 0.0f;
-#pragma unroll
-        for (int r = 0; r < MOE_MAX_TOPK; r++)
-            if (r < K) tot = tot + pk[r];
-        if (lane < K) rw[t * K + lane] = __fdiv_rn(selp[wave][lane], tot);
-        __builtin_amdgcn_wave_barrier();
     }
+    if (!ra.lists) return;
     __syncthreads();
     for (int s = tid; s < T * K; s += 64 * ROUTE_WAVES) atomicAdd(&cnt[sid[s]], 1);
     __syncthreads();
@@ -218,24 +214,33 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void k_moe_route(RouteArgs ra) {
             const int e = 4 * lane + q;
             if (e < E) {
                 beg[e] = off;
-                if (c[q]) {
-                    // problem number: experts with more vectors first (then
-                    // ascending index), so the longest workgroups start first
-                    int j = 0;
-                    for (int f = 0; f < E; f++) {
-                        const int cf = cnt[f];
-                        j += cf > c[q] || (cf == c[q] && f < e);
-                    }
-                    act_e[j] = e;
-                    vbeg[j] = off;
-                    vcnt[j] = c[q];
-                }
                 off += c[q];
             }
         }
         if (lane == 63) ra.n_act[l] = pnz;
     }
     __syncthreads();
+    {
+        // problem number: experts with more vectors first (then ascending
+        // index), so the longest workgroups start first; 4 threads per expert
+        // compare it with a quarter of the others each
+        const int e = tid >> 2, quarter = tid & 3, mine = cnt[e];
+        int j = 0;
+#pragma unroll
+        for (int f4 = 0; f4 < MOE_MAX_EXPERTS / 16; f4++) {
+            const int f = quarter * (MOE_MAX_EXPERTS / 4) + 4 * f4;
+            const int4 c = *(const int4*)&cnt[f];
+            j += (c.x > mine || (c.x == mine && f < e)) + (c.y > mine || (c.y == mine && f + 1 < e)) +
+                 (c.z > mine || (c.z == mine && f + 2 < e)) + (c.w > mine || (c.w == mine && f + 3 < e));
+        }
+        j += lane_xor_int<1>(j);
+        j += lane_xor_int<2>(j);
+        if (mine && quarter == 0) {
+            act_e[j] = e;
+            vbeg[j] = beg[e];
+            vcnt[j] = mine;
+        }
+    }
     for (int s = tid; s < T * K; s += 64 * ROUTE_WAVES) {
         const int e = sid[s];
         slots[beg[e] + atomicAdd(&fill[e], 1)] = s;
@@ -435,8 +440,12 @@ lq8_status enqueue_forward(lq8_moe* m, float* d_hidden, const float* d_scores, c
     const int max_probs = std::min(E, T * K);
     lq8_status st;
     // the router reads only the given scores: every layer's routing in one launch
-    RouteArgs ra{d_scores, T, E, K, B, m->rids, m->rw, m->n_act, m->act_e, m->vbeg, m->vcnt, m->slots};
-    hipLaunchKernelGGL(k_moe_route, dim3((unsigned)m->layers.size()), dim3(64 * ROUTE_WAVES), 0, s, ra);
+    RouteArgs ra{d_scores, T, E, K, B, m->rids, m->rw, m->n_act, m->act_e, m->vbeg, m->vcnt, m->slots, 1};
+    // one token on the batch-1 kernels: they read the ranks, not the lists
+    if (T == 1 && moe_gate_up1_supported(K, I, H) && moe_down_combine_supported(K, I)) ra.lists = 0;
+    const dim3 rgrid((unsigned)m->layers.size()), rwg(64 * ROUTE_WAVES);
+    if (E <= 128) hipLaunchKernelGGL(k_moe_route<2>, rgrid, rwg, 0, s, ra);
+    else hipLaunchKernelGGL(k_moe_route<4>, rgrid, rwg, 0, s, ra);
     LQ8_HIP(hipGetLastError());
     bool prequant = false;  // T > 1: the previous layer's combine wrote this layer's q|k|v operand
     for (size_t l = 0; l < m->layers.size(); l++) {
