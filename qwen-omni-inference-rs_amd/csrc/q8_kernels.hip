@@ -567,6 +567,8 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
+typedef float v32f __attribute__((ext_vector_type(32)));
+
 constexpr int RSRC_CFG = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
 
 struct GemmArgs {
@@ -576,7 +578,7 @@ struct GemmArgs {
     const uint16_t* ws; // weight scales (f16 bits)
     float* y;
     const float* resid;
-    int m, n, nb, np, groups, ntm, ntiles;
+    int m, n, nb, np, groups, ntm, ntn, wtiles, ntiles;  // wtiles: 16-row tiles of the weight
     int xq_bytes, xs_bytes, wc_bytes, ws_bytes;
 };
 
@@ -918,6 +920,172 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3))) voi
     }
 }
 
+// ---- GEMM of many tiles: operands shared through LDS ------------------------
+//
+// One (64 TM) x (64 TN) output block per workgroup of 2 x 2 waves, (32 TM) x
+// (32 TN) each.  A stage is PS block pairs (64 of k each): the workgroup copies
+// the 1 KiB code chunks of its 16-row tiles to LDS as they are stored (a chunk
+// per wave instruction, no registers), two stages deep; each wave reads its
+// fragments (row l % 32, half l / 32 of the block; 256-byte runs, no bank
+// conflicts) before it starts the copy of the next stage, so the copy runs
+// behind the whole stage's compute.  Per (tile, block) the arithmetic and the
+// order are k_gemm's: I_b from one v_mfma_i32_32x32x32_i8, a_g = fmaf((float)I_b,
+// dw dx, a_g), y = y + a_g after each 8 blocks.  The scale products of both
+// blocks of the pair come from one v_mfma_f32_32x32x4f16 of two blocks (lanes
+// 0..31 the scales of block 2p, lanes 32..63 of block 2p + 1, element 0 of four;
+// exact).
+// What bounds it: the conversions and fmas of that chain, 32 VALU instructions
+// per tile and block against 64 cycles of the matrix cores; with the rest of
+// the loop its VALUs issue 87% of the cycles (and the clock sits near 2.05 GHz).
+// M 4096, N 19456, K 2560 with the activation quantizer: 1060 -> 555 us (735
+// TFLOP/s) against one 32 x 32 tile per workgroup fed from L2 (k_gemm).  Back to
+// back in one run, other forms of it: 64 x 128 blocks (<1, 2, 1>, three waves per
+// SIMD) 520 us, 128 x 128 (two) 556, <1, 1, 2> 547; with the f32 scale product
+// (v_mfma_f32_32x32x1) 569, a bias in the int32 accumulators and a subtraction for
+// the conversion 712, the next step's matrix products issued between this one's
+// sums 535.
+__device__ __forceinline__ void copy_chunk_lds(__amdgpu_buffer_rsrc_t r, int8_t* dst, int voff, int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
+}
+
+template <int TM, int TN, int PS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_lds(GemmArgs g) {
+    constexpr int NA = 4 * TM, NB = 4 * TN;  // 16-row tiles of the block
+    __shared__ __attribute__((aligned(1024))) int8_t buf[2][PS][(NA + NB) * 1024];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = w & 1, wn = w >> 1;
+    const int nbm = (g.ntm + 2 * TM - 1) / (2 * TM), nbn = (g.ntn + 2 * TN - 1) / (2 * TN);
+    // each XCD (workgroup ids congruent mod 8) takes a contiguous run of blocks,
+    // numbered with up to 8 m-blocks innermost, then the n-blocks: its L2 holds
+    // those 8 m-blocks' activations while the weights stream
+    const int wgi = blockIdx.x, per = g.ntiles >> 3, rem = g.ntiles & 7, xcd = wgi & 7, j8 = wgi >> 3;
+    const int tl = xcd < rem ? xcd * (per + 1) + j8 : rem * (per + 1) + (xcd - rem) * per + j8;
+    const int mg = tl / (8 * nbn), in = tl - mg * 8 * nbn, gm = min(8, nbm - 8 * mg);
+    const int bn = in / gm, bm = mg * 8 + in - bn * gm;
+    const int half = lane >> 5, r32 = lane & 31;
+    const int nb = g.nb, np = g.np;
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc((void*)g.xq, (short)0, g.xq_bytes, RSRC_CFG);
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc((void*)g.wc, (short)0, g.wc_bytes, RSRC_CFG);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc((void*)g.xs, (short)0, g.xs_bytes, RSRC_CFG);
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc((void*)g.ws, (short)0, g.ws_bytes, RSRC_CFG);
+    // tiles past the matrix read its last tile again and are not stored
+    int sa[TM], sb[TN], ox[TM], ow[TN], mts[TM], nts[TN];
+#pragma unroll
+    for (int t = 0; t < TM; t++) {
+        sa[t] = min(bm * NA + 4 * t + w, 2 * g.ntm - 1) * np * 1024;
+        mts[t] = (bm * 2 + wm) * TM + t;
+        ox[t] = (min(mts[t], g.ntm - 1) * 2 * g.groups * 64 + r32) * 16 + half * 4;
+    }
+#pragma unroll
+    for (int t = 0; t < TN; t++) {
+        sb[t] = min(bn * NB + 4 * t + w, g.wtiles - 1) * np * 1024;
+        nts[t] = (bn * 2 + wn) * TN + t;
+        ow[t] = (min(nts[t] * 2 + (r32 >> 4), g.wtiles - 1) * 2 * np * 16 + (r32 & 15)) * 2 + half * 32;
+    }
+    const int frag = (r32 >> 4) * 1024 + half * 256 + (r32 & 15) * 16;
+    uint32_t dxn[PS][TM], dwn[PS][TN];  // the next stage's scales (f16 bits)
+    auto load_stage = [&](int p0, int into) {
+#pragma unroll
+        for (int i = 0; i < PS; i++) {
+            const int q = p0 + i, p = min(q, np - 1);  // codes past the last pair: read again, under zero scales
+#pragma unroll
+            for (int t = 0; t < TM; t++)
+                dxn[i][t] = __builtin_amdgcn_raw_buffer_load_b32(rx, ox[t], (q >> 1) * 1024 + (q & 1) * 8, 0);
+#pragma unroll
+            for (int t = 0; t < TN; t++) dwn[i][t] = __builtin_amdgcn_raw_buffer_load_b16(rw, ow[t], p * 64, 0);
+            int8_t* d = buf[into][i];
+#pragma unroll
+            for (int t = 0; t < TM; t++) copy_chunk_lds(ra, d + (4 * t + w) * 1024, lane * 16, sa[t] + p * 1024);
+#pragma unroll
+            for (int t = 0; t < TN; t++) copy_chunk_lds(rb, d + (NA + 4 * t + w) * 1024, lane * 16, sb[t] + p * 1024);
+        }
+    };
+    const v16i zi = {0};
+    const v32f zf = {0};
+    float y[TM * TN][16];
+#pragma unroll
+    for (int t = 0; t < TM * TN; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) y[t][r] = 0.0f;
+    load_stage(0, 0);
+    for (int p0 = 0; p0 < np; p0 += GEMM_GROUP / 2) {
+        float acc[TM * TN][16];
+#pragma unroll
+        for (int t = 0; t < TM * TN; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < GEMM_GROUP / 2; j += PS) {
+            const int ps = p0 + j, at = (j / PS + (PS == 4 ? p0 >> 2 : 0)) & 1;
+            if (ps >= np) break;
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the stage is in LDS
+            __syncthreads();                     // everybody's is; and the other buffer is read
+            v4i A[PS][TM][2], B[PS][TN][2];
+            uint32_t dx[PS][TM], dw[PS][TN];
+#pragma unroll
+            for (int i = 0; i < PS; i++) {
+                const int8_t* d = buf[at][i];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+#pragma unroll
+                    for (int t = 0; t < TM; t++)
+                        A[i][t][h] = *(const v4i*)(d + (wm * TM + t) * 2048 + h * 512 + frag);
+#pragma unroll
+                    for (int t = 0; t < TN; t++)
+                        B[i][t][h] = *(const v4i*)(d + NA * 1024 + (wn * TN + t) * 2048 + h * 512 + frag);
+                }
+#pragma unroll
+                for (int t = 0; t < TM; t++) dx[i][t] = dxn[i][t];
+#pragma unroll
+                for (int t = 0; t < TN; t++) dw[i][t] = 2 * (ps + i) + half < nb ? dwn[i][t] : 0u;  // past nb: zero scales
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (ps + PS < np) load_stage(ps + PS, at ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < PS; i++)
+#pragma unroll
+                for (int tm = 0; tm < TM; tm++)
+#pragma unroll
+                    for (int tn = 0; tn < TN; tn++) {
+                        float* a = acc[tm * TN + tn];
+                        const v16i I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][tm][0], B[i][tn][0], zi, 0, 0, 0);
+                        const v32f P = __builtin_amdgcn_mfma_f32_32x32x4f16(
+                            __builtin_bit_cast(v4h, make_uint2(dx[i][tm], 0u)),
+                            __builtin_bit_cast(v4h, make_uint2(dw[i][tn], 0u)), zf, 0, 0, 0);
+                        const v16i I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][tm][1], B[i][tn][1], zi, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 16; r++) a[r] = fmaf((float)I0[r], P[r], a[r]);
+#pragma unroll
+                        for (int r = 0; r < 16; r++) a[r] = fmaf((float)I1[r], P[16 + r], a[r]);
+                    }
+        }
+#pragma unroll
+        for (int t = 0; t < TM * TN; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) y[t][r] = y[t][r] + acc[t][r];
+    }
+#pragma unroll
+    for (int tn = 0; tn < TN; tn++) {
+        const int col = nts[tn] * 32 + r32;
+        if (col >= g.n) continue;
+#pragma unroll
+        for (int tm = 0; tm < TM; tm++) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int row = mts[tm] * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+                if (row < g.m) {
+                    const size_t off = (size_t)row * g.n + col;
+                    float v = y[tm * TN + tn][i];
+                    if (g.resid) v = g.resid[off] + v;
+                    g.y[off] = v;
+                }
+            }
+        }
+    }
+}
+
 // ---- small-M GEMM: 16 x 16 output tiles (v_mfma_i32_16x16x32_i8) -----------
 //
 // For few 32 x 32 tiles (M of a batch of sequences): one 16 (rows of x) x 16
@@ -1189,6 +1357,8 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
     // groups or waves the single tile measured faster (M = 512 gate/up 8.6
     // against 8.7 us; M = 128 - 256 by 1 - 2 us).
     const int ntn = (g.n + 31) / 32;
+    g.ntn = ntn;
+    g.wtiles = (int)w->tiles;
     const size_t tiles = (size_t)g.ntm * ntn;
     if (tiles > lim) return fail(LQ8_ERR_SHAPE_MISMATCH, "gemm: too many tiles");
     g.ntiles = (int)tiles;
@@ -1210,6 +1380,23 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
             default: return fail(LQ8_ERR_DEVICE, "gemm: no 16 x 16 kernel for this split");
         }
 #undef LQ8_GEMM16_CASE
+        LQ8_HIP(hipGetLastError());
+        return LQ8_OK;
+    }
+    // From 2048 32 x 32 tiles on (eight per CU) the operands are shared through LDS:
+    // 64 x 64 blocks, from 12288 tiles on 64 x 128.  Per call with the activation
+    // quantizer, other kernels -> 64 x 64 -> 64 x 128 (us): 1408 tiles (M 700, N
+    // 2048, K 2048 / 6144) 19.7 -> 21.8 -> 27.8 / 42.5 -> 48.0 -> 66.3; 2048 tiles (M
+    // 1024) 26.8 -> 22.0 -> 28.0 / 61.8 -> 50.7 -> 66.3; 2048 and 3072 tiles of K
+    // 1024 even with the others (14.2 -> 14.1, 17.1 -> 17.4); 4096 tiles (M 1024, N
+    // 4096, K 2048) 39.4 -> 33.2 -> 34.3; 8448 tiles 68.3 -> 60.3 -> 61.9; 12288
+    // tiles (K 2048 / 1024) 96.9 -> 78.9 -> 76.7 / 50.1 -> 46.0 -> 44.7.
+    if (tiles >= 2048) {
+        const int tn = tiles >= 12288 ? 2 : 1;
+        g.ntiles = ((g.ntm + 1) / 2) * ((ntn + 2 * tn - 1) / (2 * tn));
+        const dim3 gridl((unsigned)g.ntiles);
+        if (tn == 2) hipLaunchKernelGGL((k_gemm_lds<1, 2, 1>), gridl, dim3(256), 0, s, g);
+        else hipLaunchKernelGGL((k_gemm_lds<1, 1, 2>), gridl, dim3(256), 0, s, g);
         LQ8_HIP(hipGetLastError());
         return LQ8_OK;
     }

@@ -1,0 +1,43 @@
+"""The GEMM of many tiles (k_gemm_lds: operands shared through LDS) against the oracle at the edges of its range: the
+smallest tile counts that take each of its block shapes, ragged rows and columns (one row or column in the last tile,
+a last block of one 32-row tile), one block, odd block and pair counts, a group of 8 blocks and one more; and f16 scales
+that are infinite, zero or subnormal beside a padding block."""
+import numpy as np
+import pytest
+
+import lq8
+import oracle
+from test_gpu_q8 import assert_parity, gemm_case, normal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (2, 65505, 32), (33, 32769, 64), (64, 32768, 96), (65, 21857, 256), (130, 13100, 288), (515, 3873, 160),
+    (1024, 2048, 320), (2047, 1025, 544),          # 64 x 64 blocks: from 2048 tiles
+    (2, 393217, 32), (97, 98300, 96), (1023, 12289, 64), (33, 196609, 288),  # 64 x 128: from 12288 tiles
+])
+def test_many_tiles_match_oracle(ctx, m, n, k):
+    y, ref = gemm_case(ctx, m, n, k, m + n + k)
+    assert_parity(y, ref)
+
+
+@pytest.mark.parametrize("n,k", [(65505, 96), (393217, 96)])
+def test_scale_edges(ctx, n, k):
+    m = 3
+    wf = normal((n, k), 0.02, 40)
+    wf[::3] *= np.float32(1e-3)   # f16 subnormal scales
+    wf[5, 32:] = 0.0              # zero blocks
+    wf[n - 1, 64:] = 9e6          # the scale overflows f16
+    x = normal((m, k), 1.0, 41)
+    x[0] *= np.float32(1e-6)
+    x[1, 64:] = 0.0
+    x[2, :32] = -9e6
+    blocks = oracle.quantize_q8_0(wf)
+    w = lq8.Q8Weight.from_blocks(ctx, blocks, n, k)
+    y = lq8.Linear.new(w).forward(x).reshape(m, n)
+    w.free()
+    ref = oracle.gemm_q8_0(blocks, n, k, x)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(y), nan)
+    assert np.array_equal(y.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
