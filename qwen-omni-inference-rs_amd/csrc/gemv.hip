@@ -279,6 +279,80 @@ struct Stage {
                                                      __fdiv_rn(n3, den));
                 }
                 __syncthreads();
+            } else if (k <= 4 * nt) {
+                // more segments, four outputs per thread: batches of ATT_CB segments;
+                // their (m_c, l_c) in LDS (in xs, which holds 128 = 2 ATT_CB floats per
+                // head and gets the outputs last), the exps of each (segment, head) on a
+                // thread of its own, the partials CU segments at a time, numerators and
+                // denominator in registers throughout.  A head's exps one after another
+                // on one thread, and one output at a time, made this staging the
+                // longest part of the kernel.  Whole decode step (sampled) at 300 / 700 /
+                // 1500 / 3990 positions: Qwen3-1.7B 1095 -> 1022, 1217 -> 1067, 1516 ->
+                // 1168, 2508 -> 1511 us; Qwen3-4B 1980 -> 1836, 2175 -> 1900, 2718 -> 2086,
+                // 4443 -> 2664 us.  Loading (m_c, l_c) with the staging's first loads cost
+                // 15 - 25 us per step at 100 positions, 8 segments at a time spilled.
+                static_assert(2 * ATT_CB <= 128, "a batch's (m_c, l_c) must fit the staged input");
+                float* ms = xs;
+                float* ls = xs + ATT_CB * H;
+                float* mrun = dens;  // [2][H]: each head's running maximum, by parity of the batch
+                const int i = 4 * min(tid, k4 - 1), h = i >> 7;
+                const float* xo = x + (size_t)h * ATT_PART_STRIDE + (i & 127);
+                const size_t seg = (size_t)H * ATT_PART_STRIDE;
+                float den = 0.0f, n0 = 0.0f, n1 = 0.0f, n2 = 0.0f, n3 = 0.0f;
+                for (int b0 = 0, par = 0; b0 < C; b0 += ATT_CB, par ^= H) {
+                    const int nbat = min(ATT_CB, C - b0), pairs = nbat * H;
+                    if (b0 > 0) {
+#pragma unroll
+                        for (int c = 0; c < CU; c++) ov4[c] = *(const float4*)(xo + min(b0 + c, C - 1) * seg);
+                    }
+                    for (int q = tid; q < pairs; q += nt) {
+                        const float* p = x + (size_t)(b0 * H + q) * ATT_PART_STRIDE;
+                        ms[q] = p[128];
+                        ls[q] = p[129];
+                    }
+                    __syncthreads();
+                    for (int q = tid; q < pairs; q += nt) {
+                        const int c = q / H, hq = q - c * H;
+                        float m = b0 == 0 ? -__builtin_huge_valf() : mrun[par + hq], mp = m, mc = m;
+                        for (int cc = 0; cc <= c; cc++) {
+                            mc = ms[cc * H + hq];
+                            mp = m;
+                            m = m > mc ? m : mc;
+                        }
+                        coef[q * 2] = expf_cr(mp - m);
+                        coef[q * 2 + 1] = expf_cr(mc - m);
+                        if (c == nbat - 1) mrun[(par ^ H) + hq] = m;
+                    }
+                    __syncthreads();
+                    for (int c0 = 0; c0 < nbat; c0 += CU) {
+                        if (c0 > 0) {
+#pragma unroll
+                            for (int c = 0; c < CU; c++) ov4[c] = *(const float4*)(xo + min(b0 + c0 + c, C - 1) * seg);
+                        }
+                        float ca[CU], cb[CU], lc[CU];
+#pragma unroll
+                        for (int c = 0; c < CU; c++) {
+                            const int q = min(c0 + c, nbat - 1) * H + h;
+                            ca[c] = coef[q * 2];
+                            cb[c] = coef[q * 2 + 1];
+                            lc[c] = ls[q];
+                        }
+#pragma unroll
+                        for (int c = 0; c < CU; c++)
+                            if (c0 + c < nbat) {
+                                den = den * ca[c] + cb[c] * lc[c];
+                                n0 = n0 * ca[c] + cb[c] * ov4[c].x;
+                                n1 = n1 * ca[c] + cb[c] * ov4[c].y;
+                                n2 = n2 * ca[c] + cb[c] * ov4[c].z;
+                                n3 = n3 * ca[c] + cb[c] * ov4[c].w;
+                            }
+                    }
+                    __syncthreads();  // (m_c, l_c) and the coefficients are read
+                }
+                if (tid < k4)
+                    *(float4*)(xs + i) = make_float4(__fdiv_rn(n0, den), __fdiv_rn(n1, den), __fdiv_rn(n2, den),
+                                                     __fdiv_rn(n3, den));
+                __syncthreads();
             } else {
             // batches of ATT_CB segments (the coefficients of one batch in LDS):
             // each head's running maximum and denominator, and each element's
@@ -342,7 +416,7 @@ struct Stage {
 #pragma unroll
                                 for (int c = 0; c < CU; c++) {
                                     const int cc = min(c0 + c, b1 - 1);
-                                    o[c] = (c0 == 0 && e0 == 0 && k > 4 * nt)
+                                    o[c] = (c0 == 0 && e0 == 0)
                                                ? ov[e][c]
                                                : x[((size_t)cc * H + h) * ATT_PART_STRIDE + d];
                                     ca[c] = coef[((cc - b0) * H + h) * 2];  // coefficients read before the chain
