@@ -470,16 +470,17 @@ __global__ __launch_bounds__(CRQ_THREADS) void k_combine_rms_quant(
     }
 }
 
-// act = silu(gate) * up of rows gu[m, 2 inter] (as k_silu_mul: silu(g) =
-// g / (1 + exp(-g)), src/tensor.rs:1978, mlp.rs:151-164) quantized straight
-// into the GEMM operand layout.  One wave per (padded row, group of 8
-// blocks): lanes 8j .. 8j + 7 hold block j of the group, 4 consecutive values
-// each (lanes 8j .. 8j + 3 half 0, 8j + 4 .. 8j + 7 half 1); the block amax
-// folds over those 8 lanes (max is exact in any order).  Rows past m repeat
-// row m - 1.
-__global__ __launch_bounds__(256) void k_silu_quantize_act(const float* __restrict__ gu, int m, int inter, int waves,
-                                                           int groups, int np, int8_t* __restrict__ codes,
-                                                           uint32_t* __restrict__ xs) {
+// Rows quantized by (row, 8 blocks): SILU: act = silu(gate) * up of rows gu[m,
+// 2 inter] (as k_silu_mul: silu(g) = g / (1 + exp(-g)), src/tensor.rs:1978,
+// mlp.rs:151-164), else the rows x[m, inter] themselves, straight into the GEMM
+// operand layout.  One wave per (padded row, group of 8 blocks): lanes 8j ..
+// 8j + 7 hold block j of the group, 4 consecutive values each (lanes 8j .. 8j + 3
+// half 0, 8j + 4 .. 8j + 7 half 1); the block amax folds over those 8 lanes (max
+// is exact in any order).  Rows past m repeat row m - 1.
+template <bool SILU>
+__global__ __launch_bounds__(256) void k_quantize_rows(const float* __restrict__ x, int m, int inter, int waves,
+                                                       int groups, int np, int8_t* __restrict__ codes,
+                                                       uint32_t* __restrict__ xs) {
     const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (gw >= waves) return;
     const int lane = threadIdx.x & 63;
@@ -487,12 +488,19 @@ __global__ __launch_bounds__(256) void k_silu_quantize_act(const float* __restri
     const int b = g * GEMM_GROUP + (lane >> 3), hf = (lane >> 2) & 1, sub = lane & 3, nb = inter >> 5;
     float q[4] = {0, 0, 0, 0};
     if (b < nb) {
-        const float* gp = gu + (size_t)min(row, m - 1) * 2 * inter + b * 32 + hf * 16 + sub * 4;
-        const float4 gv = *(const float4*)gp, uv = *(const float4*)(gp + inter);
-        q[0] = __fdiv_rn(gv.x, 1.0f + expf_cr(-gv.x)) * uv.x;
-        q[1] = __fdiv_rn(gv.y, 1.0f + expf_cr(-gv.y)) * uv.y;
-        q[2] = __fdiv_rn(gv.z, 1.0f + expf_cr(-gv.z)) * uv.z;
-        q[3] = __fdiv_rn(gv.w, 1.0f + expf_cr(-gv.w)) * uv.w;
+        const float* gp = x + (size_t)min(row, m - 1) * (SILU ? 2 : 1) * inter + b * 32 + hf * 16 + sub * 4;
+        const float4 gv = *(const float4*)gp;
+        q[0] = gv.x;
+        q[1] = gv.y;
+        q[2] = gv.z;
+        q[3] = gv.w;
+        if (SILU) {
+            const float4 uv = *(const float4*)(gp + inter);
+            q[0] = __fdiv_rn(gv.x, 1.0f + expf_cr(-gv.x)) * uv.x;
+            q[1] = __fdiv_rn(gv.y, 1.0f + expf_cr(-gv.y)) * uv.y;
+            q[2] = __fdiv_rn(gv.z, 1.0f + expf_cr(-gv.z)) * uv.z;
+            q[3] = __fdiv_rn(gv.w, 1.0f + expf_cr(-gv.w)) * uv.w;
+        }
     }
     put_act_quarter(codes, xs, np, 2 * groups, nb, row, b, hf, sub, q);
 }
@@ -1238,6 +1246,21 @@ lq8_status launch_quantize_act(hipStream_t s, const float* x, int m, int k, int8
     const int groups = (k / 32 + GEMM_GROUP - 1) / GEMM_GROUP;
     const size_t waves = (size_t)((m + 31) / 32) * 2 * (4 * groups);
     if (!waves) return LQ8_OK;
+    // Up to one wave per SIMD of the tile-shaped kernel (a lane quantizes 16
+    // values and stores them at once), its chain per wave is what counts and four
+    // times the waves of 4 values per lane finish earlier; beyond, the whole
+    // 1 KiB chunks it stores are the better.  Linear calls (us), tile-shaped ->
+    // by rows: 144 waves (M 37, K 2080) 11.2 -> 10.5, 384 (M 128, K 3072) 9.5 ->
+    // 8.8, 512 (M 512, K 1024) 11.1 -> 10.7, 720 9.8 -> 9.4, 1024 (M 4096, K 64) 8.4
+    // -> 8.0; 1536 (M 512, K 3072) 13.3 -> 13.3, 2048 13.4 -> 13.7, 6144 (M 1024, K
+    // 6144) 26.4 -> 29.8, 10240 30.9 -> 37.7.
+    if (waves <= 1024) {
+        const size_t rw = (size_t)((m + 31) / 32 * 32) * groups;
+        hipLaunchKernelGGL(k_quantize_rows<false>, dim3(grid1(rw, 4)), dim3(256), 0, s, x, m, k, (int)rw, groups,
+                           (k / 32 + 1) / 2, codes, scales);
+        LQ8_HIP(hipGetLastError());
+        return LQ8_OK;
+    }
     // two waves per workgroup: at M = 512 the gate/up and down operands end
     // to end 12.20 -> 12.09 and 13.89 -> 13.41 us against four
     hipLaunchKernelGGL(k_quantize_act, dim3(grid1(waves, 2)), dim3(128), 0, s, x, m, k, (int)waves, 4 * groups,
@@ -1284,7 +1307,7 @@ lq8_status launch_silu_quantize_act(hipStream_t s, const float* gu, int m, int i
     const int nb = inter / 32, np = (nb + 1) / 2, groups = (nb + GEMM_GROUP - 1) / GEMM_GROUP;
     const size_t waves = (size_t)((m + 31) / 32 * 32) * groups;
     if (waves > (size_t)INT32_MAX) return fail(LQ8_ERR_SHAPE_MISMATCH, "silu_quantize_act: too many rows");
-    hipLaunchKernelGGL(k_silu_quantize_act, dim3(grid1(waves, 4)), dim3(256), 0, s, gu, m, inter, (int)waves, groups,
+    hipLaunchKernelGGL(k_quantize_rows<true>, dim3(grid1(waves, 4)), dim3(256), 0, s, gu, m, inter, (int)waves, groups,
                        np, codes, scales);
     LQ8_HIP(hipGetLastError());
     return LQ8_OK;
@@ -1384,15 +1407,22 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
         LQ8_HIP(hipGetLastError());
         return LQ8_OK;
     }
-    // From 2048 32 x 32 tiles on (eight per CU) the operands are shared through LDS:
-    // 64 x 64 blocks, from 12288 tiles on 64 x 128.  Per call with the activation
-    // quantizer, other kernels -> 64 x 64 -> 64 x 128 (us): 1408 tiles (M 700, N
-    // 2048, K 2048 / 6144) 19.7 -> 21.8 -> 27.8 / 42.5 -> 48.0 -> 66.3; 2048 tiles (M
-    // 1024) 26.8 -> 22.0 -> 28.0 / 61.8 -> 50.7 -> 66.3; 2048 and 3072 tiles of K
-    // 1024 even with the others (14.2 -> 14.1, 17.1 -> 17.4); 4096 tiles (M 1024, N
-    // 4096, K 2048) 39.4 -> 33.2 -> 34.3; 8448 tiles 68.3 -> 60.3 -> 61.9; 12288
-    // tiles (K 2048 / 1024) 96.9 -> 78.9 -> 76.7 / 50.1 -> 46.0 -> 44.7.
-    if (tiles >= 2048) {
+    // Many 32 x 32 tiles: operands shared through LDS, in 64 x 64 blocks, from
+    // 12288 tiles on 64 x 128.  Per call with the activation quantizer, other
+    // kernels -> 64 x 64 -> 64 x 128 (us): 1408 tiles (M 700, N 2048, K 2048 / 6144)
+    // 19.7 -> 21.8 -> 27.8 / 42.5 -> 48.0 -> 66.3; 2048 tiles (M 1024) 26.8 -> 22.0 ->
+    // 28.0 / 61.8 -> 50.7 -> 66.3; 4096 tiles (M 1024, N 4096, K 2048) 39.4 -> 33.2 ->
+    // 34.3; 8448 tiles 68.3 -> 60.3 -> 61.9; 12288 tiles (K 2048 / 1024) 96.9 -> 78.9
+    // -> 76.7 / 50.1 -> 46.0 -> 44.7.  Few rows share little and wait for the
+    // weights: from 12 m-tiles on (M 300: N 7000, K 1024 14.3 -> 16.0; M 512, K 256
+    // 10.6 -> 9.0), or 4 where the tiles are 12288 (M 100, N 151936, K 1024 75.9 ->
+    // 65.2; M 96, N 60000 29.3 -> 33.4; M 20, N 151936 29.4 -> 38.8).  Against a wave
+Against a wave
+    // per group (k_gemm_one) at 2 to 4 groups below 64 m-tiles: from 8192 tiles (M
+    // 1024, N 2048, K 1024 14.6 -> 14.8; M 512: N 4096, K 512 10.6 -> 10.7, N 6144, K
+    // 1024 17.1 -> 17.4; M 2048, N 1024, K 1024 17.1 -> 15.6).
+    const bool one_even = g.groups >= 2 && g.groups <= 4 && g.ntm < 64;
+    if (tiles >= 12288 ? g.ntm >= 4 : g.ntm >= 12 && tiles >= (one_even ? 8192u : 2048u)) {
         const int tn = tiles >= 12288 ? 2 : 1;
         g.ntiles = ((g.ntm + 1) / 2) * ((ntn + 2 * tn - 1) / (2 * tn));
         const dim3 gridl((unsigned)g.ntiles);

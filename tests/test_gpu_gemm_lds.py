@@ -13,18 +13,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (2, 65505, 32), (33, 32769, 64), (64, 32768, 96), (65, 21857, 256), (130, 13100, 288), (515, 3873, 160),
-    (1024, 2048, 320), (2047, 1025, 544),          # 64 x 64 blocks: from 2048 tiles
-    (2, 393217, 32), (97, 98300, 96), (1023, 12289, 64), (33, 196609, 288),  # 64 x 128: from 12288 tiles
+    (353, 5441, 32), (383, 5473, 64), (513, 3841, 96), (1023, 2049, 256), (1024, 2048, 320), (2047, 1025, 544),
+    (2049, 1000, 1024), (1025, 3940, 1056),           # 64 x 64 blocks: from 12 m-tiles and 2048 tiles
+    (97, 98273, 32), (129, 78625, 96), (1023, 12289, 64), (2049, 6049, 288),  # 64 x 128: 4 m-tiles, 12288 tiles
+    (33, 32769, 64), (2, 65505, 96), (352, 5985, 64),  # below 12 m-tiles: the other kernels
 ])
 def test_many_tiles_match_oracle(ctx, m, n, k):
     y, ref = gemm_case(ctx, m, n, k, m + n + k)
     assert_parity(y, ref)
 
 
-@pytest.mark.parametrize("n,k", [(65505, 96), (393217, 96)])
-def test_scale_edges(ctx, n, k):
-    m = 3
+@pytest.mark.parametrize("m,n,k", [(354, 5441, 96), (98, 98273, 96)])
+def test_scale_edges(ctx, m, n, k):
     wf = normal((n, k), 0.02, 40)
     wf[::3] *= np.float32(1e-3)   # f16 subnormal scales
     wf[5, 32:] = 0.0              # zero blocks

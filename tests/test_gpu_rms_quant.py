@@ -1,11 +1,12 @@
-"""RMSNorm fused into the activation quantizer (k_rms_quantize_act, a workgroup per row) at the edges of its two widths:
-one block, odd block counts, 1024 and one block more, the largest width, and row counts around the 32-row padding."""
+"""The activation quantizers at their edges.  RMSNorm fused (k_rms_quantize_act, a workgroup per row): one block, odd
+block counts, 1024 and one block more, the largest width, and row counts around the 32-row padding.  Plain rows: both
+kernels (by rows up to 1024 waves of the tile-shaped one), odd block counts, one row, and 1024 waves and the next."""
 import numpy as np
 import pytest
 
 import lq8
 import oracle
-from test_gpu_q8 import act_operand, assert_blocks_equal, normal
+from test_gpu_q8 import act_operand, assert_blocks_equal, edge_blocks, normal
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +20,14 @@ def test_rms_quantize_widths(ctx, m, k):
     w = (1.0 + 0.1 * normal(k, 1.0, k)).astype(np.float32)
     ref = oracle.quantize_q8_0(oracle.rms_norm(x, w, 1e-6))
     assert_blocks_equal(act_operand(ctx, lq8.ACT_RMSNORM, x, m, k, w), ref)
+
+
+@pytest.mark.parametrize("m,k", [(1, 32), (2, 288), (33, 2080), (31, 12256), (512, 2048), (513, 2048), (1100, 1056),
+                                 (4096, 256), (4097, 224)])
+def test_plain_quantize_kernels(ctx, m, k):
+    x = normal((m, k), 1.0, 13 * k + m)
+    x[m - 1, : k // 2] = 0.0
+    e = edge_blocks()
+    if x.size >= e.size:
+        x.reshape(-1)[x.size - e.size:] = e.reshape(-1)
+    assert_blocks_equal(act_operand(ctx, lq8.ACT_PLAIN, x, m, k), oracle.quantize_q8_0(x))
