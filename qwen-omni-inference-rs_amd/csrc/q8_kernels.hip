@@ -1417,7 +1417,6 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
     // weights: from 12 m-tiles on (M 300: N 7000, K 1024 14.3 -> 16.0; M 512, K 256
     // 10.6 -> 9.0), or 4 where the tiles are 12288 (M 100, N 151936, K 1024 75.9 ->
     // 65.2; M 96, N 60000 29.3 -> 33.4; M 20, N 151936 29.4 -> 38.8).  Against a wave
-Against a wave
     // per group (k_gemm_one) at 2 to 4 groups below 64 m-tiles: from 8192 tiles (M
     // 1024, N 2048, K 1024 14.6 -> 14.8; M 512: N 4096, K 512 10.6 -> 10.7, N 6144, K
     // 1024 17.1 -> 17.4; M 2048, N 1024, K 1024 17.1 -> 15.6).
