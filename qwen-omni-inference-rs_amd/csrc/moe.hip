@@ -150,11 +150,14 @@ __global__ __launch_bounds__(64 * ROUTE_WAVES) void k_moe_route(RouteArgs ra) {
             }
         }
         acc = wave_sum64(acc);
-        // p >= 0, so its bits order as integers; -1: no entry, or picked
+        // p >= 0 or NaN (then every p of the row is), so its bits order as
+        // integers once the NaNs have the same ones; -1: no entry, or picked
         int key[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
-            key[j] = lane + 64 * j < E ? __float_as_int(__fdiv_rn(p[j], acc)) & 0x7FFFFFFF : -1;
+        for (int j = 0; j < NJ; j++) {
+            const float q = __fdiv_rn(p[j], acc);
+            key[j] = lane + 64 * j >= E ? -1 : q == q ? __float_as_int(q) & 0x7FFFFFFF : 0x7FC00000;
+        }
         float mine = 0.0f, tot = 0.0f;  // lane r: p of rank r
         int id = 0;
         for (int r = 0; r < K; r++) {
