@@ -320,8 +320,8 @@ __global__ __launch_bounds__(256) void k_quantize_act(const float* __restrict__ 
 // agree and need no second barrier), then each thread norms and quantizes what
 // it holds (8 neighbouring threads are one block).  dim <= 1024 J.
 // A row's chain of instructions bounds it (a wave alone issues one in about 8
-// cycles): a row per wave, each lane quantizing 16 values, took
-// 5.2 us for 128 rows of 1024 (now 3.5) and 9.3 us for 1024 rows of 2048 (8.7).
+// cycles), so it is the kernel for rows that leave SIMDs with few waves; the
+// rule and the times of both kernels stand at launch_rms_quantize_act.
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int J>
@@ -367,6 +367,60 @@ __global__ __launch_bounds__(256) void k_rms_quantize_act(const float* __restric
             q[3] = bf16_round((v[j].w * inv) * bf16_round(wn[j].w));
         }
         put_act_quarter(codes, xs, np, nbp >> 2, dim >> 5, row, blk, hf, sub, q);
+    }
+}
+
+// The same for many rows: one wave per padded row, nothing of a row done twice
+// and no thread idle on a narrow one.  Lane l holds elements l, l + 64, ... in
+// registers for the sum, the normed row is staged in LDS, then lane l quantizes
+// half-blocks l, l + 64, ... (16 consecutive values each; the two halves of a
+// block are neighbouring lanes).  dim <= 64 U.
+template <int U>
+__global__ __launch_bounds__(256) void k_rms_quantize_waves(const float* __restrict__ x, const float* __restrict__ w,
+                                                            int m, int dim, float eps, int np, int nbp,
+                                                            int8_t* __restrict__ codes, uint32_t* __restrict__ xs) {
+    __shared__ __attribute__((aligned(16))) float rowbuf[4][64 * U];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int row = blockIdx.x * 4 + wv;  // the grid covers the padded rows exactly
+    const float* xr = x + (size_t)min(row, m - 1) * dim;
+    float v[U], wn[U];  // the norm weights are loaded with the row, off the sum's critical path
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        v[u] = xr[min(lane + 64 * u, dim - 1)];
+        wn[u] = w[min(lane + 64 * u, dim - 1)];
+    }
+    float acc = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (lane + 64 * u < dim) {
+            const float b = bf16_round(v[u]);
+            acc = acc + b * b;
+        }
+    acc = wave_sum64(acc);
+    const float inv = __fdiv_rn(1.0f, __builtin_sqrtf(__fdiv_rn(acc, (float)dim) + eps));
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int i = lane + 64 * u;
+        if (i < dim) rowbuf[wv][i] = bf16_round((bf16_round(v[u]) * inv) * bf16_round(wn[u]));
+    }
+    __syncthreads();
+    const int nb = dim >> 5, nhb = 2 * nbp;
+    for (int hb0 = 0; hb0 < nhb; hb0 += 64) {
+        const int hb = hb0 + lane, b = hb >> 1, hf = hb & 1;
+        float q[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        if (b < nb) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float4 t = *(const float4*)&rowbuf[wv][b * 32 + hf * 16 + 4 * i];
+                q[4 * i] = t.x;
+                q[4 * i + 1] = t.y;
+                q[4 * i + 2] = t.z;
+                q[4 * i + 3] = t.w;
+            }
+        }
+        float amax = half_amax(q);
+        amax = fmaxf(amax, lane_xor<1>(amax));
+        if (hb < nhb) put_act_half(codes, xs, np, nbp >> 2, nb, row, b, hf, q, amax);
     }
 }
 
@@ -1276,9 +1330,26 @@ lq8_status launch_rms_quantize_act(hipStream_t s, const float* x, const float* w
     if (!rms_quantize_supported(dim)) return fail(LQ8_ERR_SHAPE_MISMATCH, "rms_quantize_act: unsupported dim");
     if (m <= 0) return LQ8_OK;
     const int nb = dim / 32, np = (nb + 1) / 2, nbp = GEMM_GROUP * ((nb + GEMM_GROUP - 1) / GEMM_GROUP);
-    const dim3 grid((unsigned)((m + 31) / 32 * 32));  // the padded rows
-    if (dim <= 1024) hipLaunchKernelGGL(k_rms_quantize_act<1>, grid, dim3(256), 0, s, x, w, m, dim, eps, np, nbp, codes, scales);
-    else hipLaunchKernelGGL(k_rms_quantize_act<2>, grid, dim3(256), 0, s, x, w, m, dim, eps, np, nbp, codes, scales);
+    // A workgroup per row up to about five rows per CU (six of more than 1024
+    // values), beyond that a wave per row.  Kernel times (us), wave per row ->
+    // workgroup per row: width 32: 64 rows 5.1 -> 3.5, 1024 4.8 -> 4.1, 1280 4.4 ->
+    // 4.4, 1536 4.3 -> 4.6, 4096 5.5 -> 7.6, 16384 12.8 -> 21.2; width 1024: 64 rows
+    // 5.3 -> 3.3, 1024 5.8 -> 5.4, 1280 6.1 -> 6.0, 1536 6.2 -> 6.7, 4096 9.7 -> 13.4,
+    // 16384 23.8 -> 36.6; width 1056: 1024 rows 8.5 -> 7.1, 1536 9.0 -> 9.0, 1792 9.6 ->
+    // 9.9, 4096 14.4 -> 16.2; width 2048: 64 rows 8.4 -> 4.4, 1536 11.0 -> 11.0, 2048
+    // 12.4 -> 13.0, 16384 46.1 -> 64.0.
+    const unsigned rows = (unsigned)((m + 31) / 32 * 32);  // the padded rows
+    const int u = (dim + 63) / 64;
+    auto run = [&](auto kernel, unsigned wgs) {
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, s, x, w, m, dim, eps, np, nbp, codes, scales);
+    };
+    if (rows <= (dim <= 1024 ? 1280u : 1536u)) {
+        if (dim <= 1024) run(k_rms_quantize_act<1>, rows);
+        else run(k_rms_quantize_act<2>, rows);
+    } else if (u <= 4) run(k_rms_quantize_waves<4>, rows / 4);
+    else if (u <= 8) run(k_rms_quantize_waves<8>, rows / 4);
+    else if (u <= 16) run(k_rms_quantize_waves<16>, rows / 4);
+    else run(k_rms_quantize_waves<32>, rows / 4);
     LQ8_HIP(hipGetLastError());
     return LQ8_OK;
 }
