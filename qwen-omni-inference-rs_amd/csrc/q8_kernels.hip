@@ -1417,6 +1417,48 @@ lq8_status launch_quantize_aos(hipStream_t s, const float* x, size_t nblocks, ui
 // us per call inside the 48-layer MoE step).
 static bool gemm16_pick(int m, int groups, size_t tiles32) { return groups <= 16 && m <= 64 && tiles32 < 512; }
 
+// Many 32 x 32 tiles: operands shared through LDS (k_gemm_lds), in 64 x 64
+// blocks, from 12288 tiles on 64 x 128.  Per call with the activation quantizer,
+// other kernels -> 64 x 64 -> 64 x 128 (us): 1408 tiles (M 700, N 2048, K 2048 /
+// 6144) 19.7 -> 21.8 -> 27.8 / 42.5 -> 48.0 -> 66.3; 2048 tiles (M 1024) 26.8 -> 22.0
+// -> 28.0 / 61.8 -> 50.7 -> 66.3; 4096 tiles (M 1024, N 4096, K 2048) 39.4 -> 33.2 ->
+// 34.3; 8448 tiles 68.3 -> 60.3 -> 61.9; 12288 tiles (K 2048 / 1024) 96.9 -> 78.9 ->
+// 76.7 / 50.1 -> 46.0 -> 44.7.  Few rows share little and wait for the weights:
+// from 12 m-tiles on (M 300: N 7000, K 1024 14.3 -> 16.0; M 512, K 256 10.6 -> 9.0),
+// or 4 where the tiles are 12288 (M 100, N 151936, K 1024 75.9 -> 65.2; M 96, N
+// 60000 29.3 -> 33.4; M 20, N 151936 29.4 -> 38.8).  Against a wave per group
+// (k_gemm_one) at 2 to 4 groups below 64 m-tiles: from 8192 tiles (M 1024, N 2048,
+// K 1024 14.6 -> 14.8; M 512: N 4096, K 512 10.6 -> 10.7, N 6144, K 1024 17.1 -> 17.4;
+// M 2048, N 1024, K 1024 17.1 -> 15.6).
+// A block pays for four tiles also where the matrix has fewer: one n-tile (M
+// 65536, N 32, K 2048 160 -> 166) and 5 m-tiles of few whole groups (M 160, N
+// 89600, K 1024 54 -> 60) stay with the others.  And a CU holds three blocks (160
+// VGPRs): the fourth runs after them, alone, and what it adds is paid back only
+// when most CUs have one.  Four blocks on the fullest CU: K 2048, 13 m-tiles, 2860
+// tiles 28.7 -> 34.0, 3536 33.5 -> 34.9, 24 m-tiles 3840 36.4 -> 36.4; K 9728 (rows
+// beyond an L2 slow the others down): 13 m-tiles, 2860 108 -> 132, 28 m-tiles 3416
+// 139 -> 137; K 1024: 65 m-tiles, 3055 21.1 -> 24.1, 127 m-tiles 3175 25.9 -> 25.8.
+// Five: 13 - 17 m-tiles at 3822 - 3876 tiles 0.93 - 0.98 of the others' speed, at 4290
+// even; seven: 5720 - 5814 0.94 - 0.99, 6318 even; three, below 24 m-tiles: 2054 -
+// 2064 0.95 - 1.01, from 2200 0.98 - 1.03 and more.  At 5 groups the other kernel
+// runs a round for one of them: 2400 tiles 22.3 -> 18.9, at four blocks 3003 23.9 ->
+// 24.6, from 3080 on 1.01 and more.
+static bool gemm_lds_pick(int nb, int groups, int ntm, int ntn) {
+    const size_t tiles = (size_t)ntm * ntn;
+    const bool few = groups >= 2 && groups <= 4;
+    if (ntn == 1) return false;
+    if (tiles >= 12288) return ntm >= 4 && !(ntm == 5 && few && nb % GEMM_GROUP == 0);
+    if (ntm < 12 || tiles < (few && ntm < 64 ? 8192u : 2048u)) return false;
+    if (groups == 1 || (few && ntm < 64)) return true;
+    const int per_cu = ((ntm + 1) / 2 * ((ntn + 1) / 2) + 255) / 256;
+    size_t least = 0;
+    if (few) least = per_cu == 4 ? 3200 : per_cu == 5 ? 4100 : 0;
+    else if (groups == 5) least = per_cu == 4 ? 3072 : 0;
+    else if (per_cu == 4) least = ntm < 32 ? 3648 : ntm < 50 ? 3328 : 0;
+    else if (ntm < 24) least = per_cu == 3 ? 2112 : per_cu == 5 ? 4000 : per_cu == 7 ? 5950 : 0;
+    return tiles >= least;
+}
+
 lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int m, const lq8_weight* w, float* y,
                        const float* resid) {
     const size_t k = w->k_in;
@@ -1478,21 +1520,7 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
         LQ8_HIP(hipGetLastError());
         return LQ8_OK;
     }
-    // Many 32 x 32 tiles: operands shared through LDS, in 64 x 64 blocks, from
-    // 12288 tiles on 64 x 128.  Per call with the activation quantizer, other
-    // kernels -> 64 x 64 -> 64 x 128 (us): 1408 tiles (M 700, N 2048, K 2048 / 6144)
-    // 19.7 -> 21.8 -> 27.8 / 42.5 -> 48.0 -> 66.3; 2048 tiles (M 1024) 26.8 -> 22.0 ->
-    // 28.0 / 61.8 -> 50.7 -> 66.3; 4096 tiles (M 1024, N 4096, K 2048) 39.4 -> 33.2 ->
-    // 34.3; 8448 tiles 68.3 -> 60.3 -> 61.9; 12288 tiles (K 2048 / 1024) 96.9 -> 78.9
-    // -> 76.7 / 50.1 -> 46.0 -> 44.7.  Few rows share little and wait for the
-    // weights: from 12 m-tiles on (M 300: N 7000, K 1024 14.3 -> 16.0; M 512, K 256
-    // 10.6 -> 9.0), or 4 where the tiles are 12288 (M 100, N 151936, K 1024 75.9 ->
-    // 65.2; M 96, N 60000 29.3 -> 33.4; M 20, N 151936 29.4 -> 38.8).  Against a wave
-    // per group (k_gemm_one) at 2 to 4 groups below 64 m-tiles: from 8192 tiles (M
-    // 1024, N 2048, K 1024 14.6 -> 14.8; M 512: N 4096, K 512 10.6 -> 10.7, N 6144, K
-    // 1024 17.1 -> 17.4; M 2048, N 1024, K 1024 17.1 -> 15.6).
-    const bool one_even = g.groups >= 2 && g.groups <= 4 && g.ntm < 64;
-    if (tiles >= 12288 ? g.ntm >= 4 : g.ntm >= 12 && tiles >= (one_even ? 8192u : 2048u)) {
+    if (gemm_lds_pick(g.nb, g.groups, g.ntm, ntn)) {
         const int tn = tiles >= 12288 ? 2 : 1;
         g.ntiles = ((g.ntm + 1) / 2) * ((ntn + 2 * tn - 1) / (2 * tn));
         const dim3 gridl((unsigned)g.ntiles);

@@ -13,14 +13,29 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (353, 5441, 32), (383, 5473, 64), (513, 3841, 96), (1023, 2049, 256), (1024, 2048, 320), (2047, 1025, 544),
+    (353, 5441, 32), (383, 5473, 64), (513, 3841, 96), (1023, 2049, 256), (1024, 2048, 1312), (2047, 1025, 544),
     (2049, 1000, 1024), (1025, 3940, 1056),           # 64 x 64 blocks: from 12 m-tiles and 2048 tiles
-    (97, 98273, 32), (129, 78625, 96), (1023, 12289, 64), (2049, 6049, 288),  # 64 x 128: 4 m-tiles, 12288 tiles
-    (33, 32769, 64), (2, 65505, 96), (352, 5985, 64),  # below 12 m-tiles: the other kernels
+    (97, 98273, 32), (129, 78625, 96), (1023, 12289, 64), (2049, 6049, 288), (160, 78656, 544),  # 64 x 128: 12288 tiles
+    (33, 32769, 64), (2, 65505, 96), (352, 5985, 64),  # few m-tiles: the other kernels
+    (1024, 2048, 320),                                 # 2 to 4 groups of blocks below 8192 tiles: the other kernels
+    (65536, 32, 64), (129, 78625, 512),                # one n-tile, 5 m-tiles of whole groups: the other kernels
 ])
 def test_many_tiles_match_oracle(ctx, m, n, k):
     y, ref = gemm_case(ctx, m, n, k, m + n + k)
     assert_parity(y, ref)
+
+
+# the last tile count of the other kernels and the first of k_gemm_lds, at 2 to 4 groups of blocks, at 5, and at more with
+# three, four, five and seven 64 x 64 blocks on the fullest CU
+@pytest.mark.parametrize("m,k,below,above", [
+    (1024, 320, 8160, 8192), (2048, 288, 1568, 1600), (2051, 288, 2016, 2048), (416, 1056, 7552, 7584),
+    (416, 1312, 5152, 5216), (410, 1312, 8960, 8992), (1248, 1312, 2720, 2752), (416, 1312, 9824, 9856),
+    (416, 1312, 14624, 14656),
+])
+def test_both_sides_of_the_tile_rule(ctx, m, k, below, above):
+    for n in (below, above):
+        y, ref = gemm_case(ctx, m, n, k, m + n + k)
+        assert_parity(y, ref)
 
 
 @pytest.mark.parametrize("m,n,k", [(354, 5441, 96), (98, 98273, 96)])
