@@ -1,7 +1,9 @@
 """Prefill attention (k_attn_rows: products on the matrix cores, outputs quantized into the o projection's operand)
 against the CPU oracle, bit for bit, where its tiles can go wrong: head groups that do not divide the 16 (or 32) query
 vectors of a workgroup, odd head counts (padding blocks of the operand), rows around the tiles and the 64-position
-segments, chunks that start inside a segment, both vector counts per workgroup, and keys and values that are not finite."""
+segments, chunks that start inside a segment, a few rows behind a long cache, both vector counts per workgroup, score
+differences over the whole range of the exp (its subnormal results and its cutoff among them), and keys and values that
+are not finite.  One case takes the GEMM of many tiles with a residual (the o and down projections of a long prompt)."""
 import numpy as np
 import pytest
 
@@ -26,13 +28,17 @@ def config(heads, kv, positions, layers=2):
 # (heads, kv heads, chunk lengths): 32 vectors per workgroup in the 64-head cases (kv heads * tiles >= 1024), else 16
 @pytest.mark.parametrize("heads,kv,chunks", [
     (2, 2, (2, 15, 17)), (3, 1, (64, 2)), (5, 5, (65,)), (7, 1, (63, 3, 130)), (6, 2, (31, 34, 64)),
-    (16, 1, (70,)), (12, 4, (100, 93)), (64, 64, (513,)), (64, 64, (40, 500)), (66, 33, (600,)),
+    (16, 1, (70,)), (12, 4, (100, 93)), (64, 64, (513,)), (64, 64, (40, 500)), (66, 33, (600,)), (2, 1, (2300, 3, 2)),
 ])
 def test_prefill_rows_match_oracle(ctx, heads, kv, chunks):
     cfg = config(heads, kv, 64 * ((sum(chunks) + 63) // 64), layers=1 if heads > 16 else 2)
     tensors = oracle.random_q8_tensors(cfg, seed=heads * 100 + kv, layer_std=0.1, norm_jitter=0.1)
+    compare_chunks(ctx, cfg, tensors, chunks)
+
+
+def compare_chunks(ctx, cfg, tensors, chunks):
     model, ref = lq8.Qwen3ForCausalLM.load(ctx, cfg, tensors), oracle.Model(cfg, tensors)
-    ids = np.random.default_rng(heads).integers(0, cfg.vocab_size, sum(chunks)).astype(np.uint32)
+    ids = np.random.default_rng(cfg.num_attention_heads).integers(0, cfg.vocab_size, sum(chunks)).astype(np.uint32)
     at = 0
     for n in chunks:
         got, want = (m.forward_with_intermediates(ids[at:at + n], at) for m in (model, ref))
@@ -41,6 +47,29 @@ def test_prefill_rows_match_oracle(ctx, heads, kv, chunks):
         at += n
     model.free()
     ref.close()
+
+
+# kv heads * tiles >= 1024 (32 vectors per workgroup) in the cases of 63 heads and more, whose groups of 3, 7 and 11 heads
+# leave spare vectors
+@pytest.mark.parametrize("heads,kv,chunks", [(4, 2, (70, 130)), (3, 1, (300,)), (66, 22, (480,)), (63, 9, (460,)),
+                                             (66, 6, (345,))])
+def test_score_differences_past_the_exp_range(ctx, heads, kv, chunks):
+    """Large q and k norm weights: scores of a row lie up to hundreds apart, so that exps of differences to the maximum
+    are subnormal (below -87.3), zero (below about -104) and past the cutoff (-110), in the first and in later segments,
+    with the running maximum rising by as much."""
+    cfg = config(heads, kv, 64 * ((sum(chunks) + 63) // 64), layers=1)
+    tensors = oracle.random_q8_tensors(cfg, seed=heads + kv, layer_std=0.1, norm_jitter=0.1)
+    tensors[4] = (tensors[4] * np.float32(6.0)).astype(np.float32)
+    tensors[5] = (tensors[5] * np.float32(6.0)).astype(np.float32)
+    compare_chunks(ctx, cfg, tensors, chunks)
+
+
+def test_long_prompt_residual_gemms(ctx):
+    """o and down of 1025 rows into 2016 columns: 33 x 63 output tiles (a ragged last row tile) at 5 and 6 groups of
+    blocks, so both run k_gemm_lds with the residual added in place."""
+    cfg = lq8.Qwen3Config(vocab_size=96, hidden_size=2016, intermediate_size=1312, num_hidden_layers=1,
+                          num_attention_heads=9, num_key_value_heads=3, head_dim=128, max_position_embeddings=1088)
+    compare_chunks(ctx, cfg, oracle.random_q8_tensors(cfg, seed=21, layer_std=0.05, norm_jitter=0.1), (1025,))
 
 
 @pytest.mark.parametrize("heads,kv,n,at", [(4, 2, 50, 40), (4, 2, 130, 70), (64, 64, 513, 500)])
