@@ -387,26 +387,20 @@ lq8_status enqueue_decode(lq8_model* m, const uint32_t* d_id, const int* d_pos, 
     return LQ8_OK;
 }
 
-lq8_status quant_gemm(lq8_model* m, const float* x, int n, const lq8_weight* w, float* y, const float* resid) {
-    hipStream_t s = m->ctx->stream;
-    uint32_t* xs = reinterpret_cast<uint32_t*>(m->P_xs);
-    lq8_status st = launch_quantize_act(s, x, n, (int)w->k_in, m->P_xq, xs);
-    if (st) return st;
-    return launch_gemm(s, m->P_xq, xs, n, w, y, resid);
-}
-
 // GEMM input RmsNorm(h) rows: the norm is fused into the activation quantizer
 // (the same operand as rms_norm_rows followed by quantize_act) where the
 // hidden size allows it.
 lq8_status norm_quant_gemm(lq8_model* m, const float* h, const float* norm_w, int n, const lq8_weight* w, float* y) {
     hipStream_t s = m->ctx->stream;
     const int Hd = (int)m->c.hidden_size;
-    if (!rms_quantize_supported(Hd)) {
-        lq8_status st = launch_rms_norm_rows(s, h, norm_w, n, Hd, m->c.rms_norm_eps, m->P_x);
-        return st ? st : quant_gemm(m, m->P_x, n, w, y, nullptr);
-    }
     uint32_t* xs = reinterpret_cast<uint32_t*>(m->P_xs);
-    lq8_status st = launch_rms_quantize_act(s, h, norm_w, n, Hd, m->c.rms_norm_eps, m->P_xq, xs);
+    lq8_status st;
+    if (rms_quantize_supported(Hd)) {
+        st = launch_rms_quantize_act(s, h, norm_w, n, Hd, m->c.rms_norm_eps, m->P_xq, xs);
+    } else {
+        st = launch_rms_norm_rows(s, h, norm_w, n, Hd, m->c.rms_norm_eps, m->P_x);
+        if (!st) st = launch_quantize_act(s, m->P_x, n, Hd, m->P_xq, xs);
+    }
     return st ? st : launch_gemm(s, m->P_xq, xs, n, w, y, nullptr);
 }
 

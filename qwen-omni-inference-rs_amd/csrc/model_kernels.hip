@@ -272,6 +272,7 @@ __device__ __forceinline__ uint2 codes8(const float (&y)[8], float id) {
 
 template <int NVT>
 __global__ __launch_bounds__(AR_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_attn_rows(AttnRowsLaunch a) {
+    static_assert(NVT == 1 || NVT == 2, "16 or 8 threads per softmax vector");
     constexpr int NV = 16 * NVT, PARTS = AR_THREADS / NV, KPT = SEG / PARTS;
     __shared__ __attribute__((aligned(16))) float qs[NV * AR_QPAD];
     __shared__ __attribute__((aligned(16))) float sbuf[2][NV * AR_SPAD];  // scores, then exps
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(AR_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
             for (int i = 0; i < KPT; i++) mc = fmaxf(mc, x[i]);
             mc = fmaxf(mc, lane_xor<1>(mc));
             mc = fmaxf(mc, lane_xor<2>(mc));
-            if (PARTS > 4) mc = fmaxf(mc, lane_xor<4>(mc));
+            mc = fmaxf(mc, lane_xor<4>(mc));
             if (PARTS > 8) mc = fmaxf(mc, lane_xor<8>(mc));
 #pragma unroll
             for (int i = 0; i < KPT; i++) x[i] = x[i] - mc;
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(AR_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
                 for (int i = 0; i < d; i++) x[i] = x[i] + x[i + d];
             float lc = x[0];
             if (PARTS > 8) lc = lc + lane_xor<8>(lc);
-            if (PARTS > 4) lc = lc + lane_xor<4>(lc);
+            lc = lc + lane_xor<4>(lc);
             lc = lc + lane_xor<2>(lc);
             lc = lc + lane_xor<1>(lc);
             const float ex = x[KPT], ey = lane_xor<1>(ex);

@@ -994,8 +994,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3))) voi
 
 // ---- GEMM of many tiles: operands shared through LDS ------------------------
 //
-// One (64 TM) x (64 TN) output block per workgroup of 2 x 2 waves, (32 TM) x
-// (32 TN) each.  A stage is PS block pairs (64 of k each): the workgroup copies
+// One 64 x (64 TN) output block per workgroup of 2 x 2 waves, 32 x (32 TN)
+// each.  A stage is PS block pairs (64 of k each): the workgroup copies
 // the 1 KiB code chunks of its 16-row tiles to LDS as they are stored (a chunk
 // per wave instruction, no registers), two stages deep; each wave reads its
 // fragments (row l % 32, half l / 32 of the block; 256-byte runs, no bank
@@ -1011,8 +1011,8 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3))) voi
 // the loop its VALUs issue 87% of the cycles (and the clock sits near 2.05 GHz).
 // M 4096, N 19456, K 2560 with the activation quantizer: 1060 -> 555 us (735
 // TFLOP/s) against one 32 x 32 tile per workgroup fed from L2 (k_gemm).  Back to
-// back in one run, other forms of it: 64 x 128 blocks (<1, 2, 1>, three waves per
-// SIMD) 520 us, 128 x 128 (two) 556, <1, 1, 2> 547; with the f32 scale product
+// back in one run, other forms of it: 64 x 128 blocks (<2, 1>, three waves per
+// SIMD) 520 us, 128 x 128 (two) 556, <1, 2> 547; with the f32 scale product
 // (v_mfma_f32_32x32x1) 569, a bias in the int32 accumulators and a subtraction for
 // the conversion 712, the next step's matrix products issued between this one's
 // sums 535.
@@ -1020,14 +1020,15 @@ __device__ __forceinline__ void copy_chunk_lds(__amdgpu_buffer_rsrc_t r, int8_t*
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
 }
 
-template <int TM, int TN, int PS>
+template <int TN, int PS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_lds(GemmArgs g) {
-    constexpr int NA = 4 * TM, NB = 4 * TN;  // 16-row tiles of the block
+    static_assert(PS == 1 || PS == 2, "a group of four pairs must end on the second buffer");
+    constexpr int NA = 4, NB = 4 * TN;  // 16-row tiles of the block
     __shared__ __attribute__((aligned(1024))) int8_t buf[2][PS][(NA + NB) * 1024];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = w & 1, wn = w >> 1;
-    const int nbm = (g.ntm + 2 * TM - 1) / (2 * TM), nbn = (g.ntn + 2 * TN - 1) / (2 * TN);
+    const int nbm = (g.ntm + 1) / 2, nbn = (g.ntn + 2 * TN - 1) / (2 * TN);
     // each XCD (workgroup ids congruent mod 8) takes a contiguous run of blocks,
     // numbered with up to 8 m-blocks innermost, then the n-blocks: its L2 holds
     // those 8 m-blocks' activations while the weights stream
@@ -1042,13 +1043,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     const auto rx = __builtin_amdgcn_make_buffer_rsrc((void*)g.xs, (short)0, g.xs_bytes, RSRC_CFG);
     const auto rw = __builtin_amdgcn_make_buffer_rsrc((void*)g.ws, (short)0, g.ws_bytes, RSRC_CFG);
     // tiles past the matrix read its last tile again and are not stored
-    int sa[TM], sb[TN], ox[TM], ow[TN], mts[TM], nts[TN];
-#pragma unroll
-    for (int t = 0; t < TM; t++) {
-        sa[t] = min(bm * NA + 4 * t + w, 2 * g.ntm - 1) * np * 1024;
-        mts[t] = (bm * 2 + wm) * TM + t;
-        ox[t] = (min(mts[t], g.ntm - 1) * 2 * g.groups * 64 + r32) * 16 + half * 4;
-    }
+    int sb[TN], ow[TN], nts[TN];
+    const int sa = min(bm * NA + w, 2 * g.ntm - 1) * np * 1024, mt = bm * 2 + wm;
+    const int ox = (min(mt, g.ntm - 1) * 2 * g.groups * 64 + r32) * 16 + half * 4;
 #pragma unroll
     for (int t = 0; t < TN; t++) {
         sb[t] = min(bn * NB + 4 * t + w, g.wtiles - 1) * np * 1024;
@@ -1056,59 +1053,53 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         ow[t] = (min(nts[t] * 2 + (r32 >> 4), g.wtiles - 1) * 2 * np * 16 + (r32 & 15)) * 2 + half * 32;
     }
     const int frag = (r32 >> 4) * 1024 + half * 256 + (r32 & 15) * 16;
-    uint32_t dxn[PS][TM], dwn[PS][TN];  // the next stage's scales (f16 bits)
+    uint32_t dxn[PS], dwn[PS][TN];  // the next stage's scales (f16 bits)
     auto load_stage = [&](int p0, int into) {
 #pragma unroll
         for (int i = 0; i < PS; i++) {
             const int q = p0 + i, p = min(q, np - 1);  // codes past the last pair: read again, under zero scales
-#pragma unroll
-            for (int t = 0; t < TM; t++)
-                dxn[i][t] = __builtin_amdgcn_raw_buffer_load_b32(rx, ox[t], (q >> 1) * 1024 + (q & 1) * 8, 0);
+            dxn[i] = __builtin_amdgcn_raw_buffer_load_b32(rx, ox, (q >> 1) * 1024 + (q & 1) * 8, 0);
 #pragma unroll
             for (int t = 0; t < TN; t++) dwn[i][t] = __builtin_amdgcn_raw_buffer_load_b16(rw, ow[t], p * 64, 0);
             int8_t* d = buf[into][i];
-#pragma unroll
-            for (int t = 0; t < TM; t++) copy_chunk_lds(ra, d + (4 * t + w) * 1024, lane * 16, sa[t] + p * 1024);
+            copy_chunk_lds(ra, d + w * 1024, lane * 16, sa + p * 1024);
 #pragma unroll
             for (int t = 0; t < TN; t++) copy_chunk_lds(rb, d + (NA + 4 * t + w) * 1024, lane * 16, sb[t] + p * 1024);
         }
     };
     const v16i zi = {0};
     const v32f zf = {0};
-    float y[TM * TN][16];
+    float y[TN][16];
 #pragma unroll
-    for (int t = 0; t < TM * TN; t++)
+    for (int t = 0; t < TN; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) y[t][r] = 0.0f;
     load_stage(0, 0);
     for (int p0 = 0; p0 < np; p0 += GEMM_GROUP / 2) {
-        float acc[TM * TN][16];
+        float acc[TN][16];
 #pragma unroll
-        for (int t = 0; t < TM * TN; t++)
+        for (int t = 0; t < TN; t++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
 #pragma unroll
         for (int j = 0; j < GEMM_GROUP / 2; j += PS) {
-            const int ps = p0 + j, at = (j / PS + (PS == 4 ? p0 >> 2 : 0)) & 1;
+            const int ps = p0 + j, at = j / PS & 1;
             if (ps >= np) break;
             __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the stage is in LDS
             __syncthreads();                     // everybody's is; and the other buffer is read
-            v4i A[PS][TM][2], B[PS][TN][2];
-            uint32_t dx[PS][TM], dw[PS][TN];
+            v4i A[PS][2], B[PS][TN][2];
+            uint32_t dx[PS], dw[PS][TN];
 #pragma unroll
             for (int i = 0; i < PS; i++) {
                 const int8_t* d = buf[at][i];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-#pragma unroll
-                    for (int t = 0; t < TM; t++)
-                        A[i][t][h] = *(const v4i*)(d + (wm * TM + t) * 2048 + h * 512 + frag);
+                    A[i][h] = *(const v4i*)(d + wm * 2048 + h * 512 + frag);
 #pragma unroll
                     for (int t = 0; t < TN; t++)
                         B[i][t][h] = *(const v4i*)(d + NA * 1024 + (wn * TN + t) * 2048 + h * 512 + frag);
                 }
-#pragma unroll
-                for (int t = 0; t < TM; t++) dx[i][t] = dxn[i][t];
+                dx[i] = dxn[i];
 #pragma unroll
                 for (int t = 0; t < TN; t++) dw[i][t] = 2 * (ps + i) + half < nb ? dwn[i][t] : 0u;  // past nb: zero scales
             }
@@ -1118,23 +1109,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
             for (int i = 0; i < PS; i++)
 #pragma unroll
-                for (int tm = 0; tm < TM; tm++)
+                for (int tn = 0; tn < TN; tn++) {
+                    float* a = acc[tn];
+                    const v16i I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][0], B[i][tn][0], zi, 0, 0, 0);
+                    const v32f P = __builtin_amdgcn_mfma_f32_32x32x4f16(
+                        __builtin_bit_cast(v4h, make_uint2(dx[i], 0u)),
+                        __builtin_bit_cast(v4h, make_uint2(dw[i][tn], 0u)), zf, 0, 0, 0);
+                    const v16i I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][1], B[i][tn][1], zi, 0, 0, 0);
 #pragma unroll
-                    for (int tn = 0; tn < TN; tn++) {
-                        float* a = acc[tm * TN + tn];
-                        const v16i I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][tm][0], B[i][tn][0], zi, 0, 0, 0);
-                        const v32f P = __builtin_amdgcn_mfma_f32_32x32x4f16(
-                            __builtin_bit_cast(v4h, make_uint2(dx[i][tm], 0u)),
-                            __builtin_bit_cast(v4h, make_uint2(dw[i][tn], 0u)), zf, 0, 0, 0);
-                        const v16i I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[i][tm][1], B[i][tn][1], zi, 0, 0, 0);
+                    for (int r = 0; r < 16; r++) a[r] = fmaf((float)I0[r], P[r], a[r]);
 #pragma unroll
-                        for (int r = 0; r < 16; r++) a[r] = fmaf((float)I0[r], P[r], a[r]);
-#pragma unroll
-                        for (int r = 0; r < 16; r++) a[r] = fmaf((float)I1[r], P[16 + r], a[r]);
-                    }
+                    for (int r = 0; r < 16; r++) a[r] = fmaf((float)I1[r], P[16 + r], a[r]);
+                }
         }
 #pragma unroll
-        for (int t = 0; t < TM * TN; t++)
+        for (int t = 0; t < TN; t++)
 #pragma unroll
             for (int r = 0; r < 16; r++) y[t][r] = y[t][r] + acc[t][r];
     }
@@ -1143,16 +1132,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const int col = nts[tn] * 32 + r32;
         if (col >= g.n) continue;
 #pragma unroll
-        for (int tm = 0; tm < TM; tm++) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int row = mts[tm] * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
-                if (row < g.m) {
-                    const size_t off = (size_t)row * g.n + col;
-                    float v = y[tm * TN + tn][i];
-                    if (g.resid) v = g.resid[off] + v;
-                    g.y[off] = v;
-                }
+        for (int i = 0; i < 16; i++) {
+            const int row = mt * 32 + 8 * (i >> 2) + 4 * half + (i & 3);
+            if (row < g.m) {
+                const size_t off = (size_t)row * g.n + col;
+                float v = y[tn][i];
+                if (g.resid) v = g.resid[off] + v;
+                g.y[off] = v;
             }
         }
     }
@@ -1524,8 +1510,8 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
         const int tn = tiles >= 12288 ? 2 : 1;
         g.ntiles = ((g.ntm + 1) / 2) * ((ntn + 2 * tn - 1) / (2 * tn));
         const dim3 gridl((unsigned)g.ntiles);
-        if (tn == 2) hipLaunchKernelGGL((k_gemm_lds<1, 2, 1>), gridl, dim3(256), 0, s, g);
-        else hipLaunchKernelGGL((k_gemm_lds<1, 1, 2>), gridl, dim3(256), 0, s, g);
+        if (tn == 2) hipLaunchKernelGGL((k_gemm_lds<2, 1>), gridl, dim3(256), 0, s, g);
+        else hipLaunchKernelGGL((k_gemm_lds<1, 2>), gridl, dim3(256), 0, s, g);
         LQ8_HIP(hipGetLastError());
         return LQ8_OK;
     }
