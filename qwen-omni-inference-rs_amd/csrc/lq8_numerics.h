@@ -67,7 +67,8 @@ constexpr int EXP_CONSTS = 14;
 // branches and side by side (the chains are long): the same steps with k
 // rounded by adding 1.5 * 2^52 (its low word is then k), so that a NaN passes
 // through; what they give below -110 (-inf included) is replaced.  c: the
-// constants, as the caller holds them.
+// constants, as the caller holds them.  Equal to expf_cr for every such x (all
+// 2^31 of them compared on the device).
 template <int N, typename P>
 __device__ __forceinline__ void expf_le0(float (&x)[N], P c) {
     double r[N], p[N];

@@ -190,8 +190,9 @@ __global__ __launch_bounds__(128) void k_attn_combine(const float* __restrict__ 
 // The chains round every product before it is added, so a multiply-accumulate
 // is no fma; the matrix cores take the products: v_mfma_f32_16x16x1_4b_f32
 // with C = 0 gives four 16 x 16 outer products, each element round(a * b)
-// exactly as v_mul_f32 rounds it (subnormals included; a zero product is +0
-// instead of -0, which no sum that starts from +0 can tell), at twice the
+// exactly as v_mul_f32 rounds it (each is fma(a, b, +0): 4e8 products over all
+// exponents, subnormal ones among them, agree; a zero factor gives +0 where a
+// multiply may give -0, which no sum that starts from +0 can tell), at twice the
 // VALU's rate, and the VALU only adds them in the order of the chain.  Operand
 // lane l is row (column) l % 16 of block l / 16, and the blocks are four terms
 // of the chain: a float4 of 16 consecutive terms per lane group feeds 4
@@ -209,15 +210,15 @@ __global__ __launch_bounds__(128) void k_attn_combine(const float* __restrict__ 
 // unless V is not finite there, and a segment where that is so takes the adds
 // one by one under the row's length.
 //
-// Bound: instruction issue.  At 2048 rows (Qwen3-0.6B) the VALU instructions
-// (758k cycles per SIMD, 540k of them the chains' adds) and the f32 matrix
-// instructions (270k; they use the same fp32 units, and issuing the next
-// group's products between a group's adds changed nothing) fill the 1.0M
-// cycles the kernel runs.  Against one chain per thread from LDS followed by
-// the separate quantizer: 1283 -> 423 us at 2048 rows, 370 -> 128 at 1024, 109
-// -> 48 at 512, 20 -> 15 at 128 (where a wave's chain latencies bound it), and
-// 5 us of quantizer less.  64 vectors per workgroup (256 VGPRs) measured 553
-// us at 2048 rows.
+// Bound: instruction issue.  For 951 rows behind 2048 positions of Qwen3-1.7B
+// the VALU instructions (840k cycles per SIMD, about 600k of them the chains'
+// adds) and the f32 matrix instructions (303k; they use the same fp32 units, and
+// issuing the next group's products between a group's adds changed nothing) fill
+// the 1.13M cycles the kernel runs (496 us).  Against one chain per thread from
+// LDS followed by the separate quantizer, per layer of Qwen3-0.6B: 1283 -> 398 us
+// at 2048 rows, 370 -> 125 at 1024, 109 -> 48 at 512, 20 -> 15 at 128 (where a
+// wave's chain latencies bound it), and 5 us of quantizer less.  64 vectors per
+// workgroup (256 VGPRs) measured 553 us at 2048 rows.
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int AR_THREADS = 256;
 constexpr int AR_QPAD = 132, AR_SPAD = 68;  // LDS row strides: 16-byte aligned, 4 banks apart
@@ -621,9 +622,11 @@ lq8_status launch_attention_rows(hipStream_t s, const AttnRowsLaunch& a) {
         return fail(LQ8_ERR_SHAPE_MISMATCH, "attention: unsupported head layout");
     const int G = a.num_heads / a.num_kv_heads;
     // 32 query vectors per workgroup where that still leaves four workgroups a
-    // CU (the per-step work is shared by more rows: 430 against 462 us at 2048
-    // rows of Qwen3-0.6B), else 16 (the rows' lengths balance better: 133
-    // against 159 us at 1024 rows, 48 against 73 at 512)
+    // CU (the per-step work is shared by more rows: 398 against 415 us at 2048
+    // rows of Qwen3-0.6B), else 16 (the rows' lengths balance better: 125
+    // against 152 us at 1024 rows, 48 against 72 at 512, 15 against 24 at 128).
+    // Behind a cache the lengths differ less and 16 loses that: 1024 rows behind
+    // 1024 positions 293 against 291, behind 2048 472 against 444
     auto tiles = [&](int nv) { return (a.n + nv / G - 1) / (nv / G); };
     const bool two = a.num_kv_heads * tiles(32) >= 1024;
     const dim3 grid((unsigned)a.num_kv_heads, (unsigned)tiles(two ? 32 : 16));

@@ -91,8 +91,10 @@ namespace {
 // One CU does a layer's routing, so instructions and serial LDS reads bound
 // it: picking by rounds (about 25 instructions per rank) instead of ranking
 // every entry against every other, and the numbering by 4 threads per expert
-// with 16-byte reads instead of one thread per 4 experts, took two layers of
-// 128 experts, top 8, from 66 to 11 us at 32 tokens and from 31 to 3.3 us at one.
+// with 16-byte reads instead of one thread per 4 experts, took a launch for 128
+// experts, top 8, from 66 to 11 us at 32 tokens and from 31 to 3.4 us at one.  It
+// is one launch per step whatever the layers (48: 12 and 3.8 us), so a stack of
+// 48 gains 1 to 2 %: 37.1 -> 36.3 us per layer at one token, 161.4 -> 160.0 at 32.
 constexpr int ROUTE_WAVES = 16;
 struct RouteArgs {
     const float* scores;  // [layers][T][E]

@@ -1007,12 +1007,12 @@ __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(3))) voi
 // 0..31 the scales of block 2p, lanes 32..63 of block 2p + 1, element 0 of four;
 // exact).
 // What bounds it: the conversions and fmas of that chain, 32 VALU instructions
-// per tile and block against 64 cycles of the matrix cores; with the rest of
-// the loop its VALUs issue 87% of the cycles (and the clock sits near 2.05 GHz).
-// M 4096, N 19456, K 2560 with the activation quantizer: 1060 -> 555 us (735
-// TFLOP/s) against one 32 x 32 tile per workgroup fed from L2 (k_gemm).  Back to
-// back in one run, other forms of it: 64 x 128 blocks (<2, 1>, three waves per
-// SIMD) 520 us, 128 x 128 (two) 556, <1, 2> 547; with the f32 scale product
+// per tile and block, 128 cycles of a SIMD against 64 of its matrix core; with
+// the rest of the loop its VALUs issue 89% of the cycles (and the clock sits near
+// 2 GHz).  M 4096, N 19456, K 2560 with the activation quantizer: 1060 -> 536 - 555
+// us (735 - 760 TFLOP/s) against one 32 x 32 tile per workgroup fed from L2
+// (k_gemm).  Back to back in one run, other forms of it: 64 x 128 blocks (<2, 1>,
+// three waves per SIMD) 520 us, 128 x 128 (two) 556, <1, 2> 547; with the f32 scale product
 // (v_mfma_f32_32x32x1) 569, a bias in the int32 accumulators and a subtraction for
 // the conversion 712, the next step's matrix products issued between this one's
 // sums 535.
@@ -1470,15 +1470,16 @@ lq8_status launch_gemm(hipStream_t s, const int8_t* xq, const uint32_t* xs, int 
     g.xs_bytes = (int)xs_bytes;
     g.wc_bytes = (int)wc_bytes;
     g.ws_bytes = (int)ws_bytes;
-    // K split over S waves (one group per wave per round).  S: every group its
-    // own wave (one round, no running sum: k_gemm_one) when the groups are
-    // few (<= 4) or the waves that gives stay <= 8192; otherwise the fewest of
-    // 2, 3, 4, 6, 8, 12, 16 that give >= 2048 waves (k_gemm, one 32 x 32 tile
-    // per workgroup, running sum over rounds).  k_gemm_one gives each wave two
-    // 32-row tiles sharing the weight fragment for long K (8 - 12 groups) when
-    // that still leaves >= 3072 waves (M = 512 down 8.0 -> 7.0 us); with fewer
-    // groups or waves the single tile measured faster (M = 512 gate/up 8.6
-    // against 8.7 us; M = 128 - 256 by 1 - 2 us).
+    // What gemm16_pick and gemm_lds_pick leave: K split over S waves (one group
+    // per wave per round).  S: every group its own wave (one round, no running
+    // sum: k_gemm_one) when the groups are few (<= 4) or the waves that gives
+    // stay <= 8192; otherwise the fewest of 2, 3, 4, 6, 8, 12, 16 that give >=
+    // 2048 waves (k_gemm, one 32 x 32 tile per workgroup, running sum over
+    // rounds).  k_gemm_one gives each wave two 32-row tiles sharing the weight
+    // fragment for long K (8 - 12 groups) when that still leaves >= 3072 waves (M
+    // = 512 down 8.0 -> 7.0 us); with fewer groups or waves the single tile
+    // measured faster (M = 512 gate/up 8.6 against 8.7 us; M = 128 - 256 by 1 - 2
+    // us).
     const int ntn = (g.n + 31) / 32;
     g.ntn = ntn;
     g.wtiles = (int)w->tiles;

@@ -106,7 +106,7 @@ def test_rmsnorm_activation_quantizer(ctx, m, k):
 
 @pytest.mark.parametrize("m,inter", [(512, 3072), (45, 800)])
 def test_silu_activation_quantizer(ctx, m, inter):
-    """k_silu_quantize_act (silu(gate) * up fused into the quantizer): the
+    """k_quantize_rows<true> (silu(gate) * up fused into the quantizer): the
     blocks of quantize(silu(g) * u), silu(g) = g / (1 + exp(-g)) with the
     oracle's exp, every step an f32 operation."""
     gu = normal((m, 2 * inter), 2.0, inter)
